@@ -61,4 +61,9 @@ bool qgemm_supported(int dtype, int sdt, int group_size, int bits, const void* x
                      const void* w, int64_t k);
 void qgemm_launch(const QgemmArgs& a, hipStream_t s);
 
+// Many rows (qgemm_tile.hip): K a multiple of 512, w 16-byte and scales and
+// biases 4-byte aligned, a block's rows and columns within 2 GiB.
+bool qgemm_tile_fits(const QgemmArgs& a);
+void qgemm_tile_launch(const QgemmArgs& a, hipStream_t s);
+
 }  // namespace hgk

@@ -4,9 +4,10 @@
 // with w [N, K/8] u32 (8 codes per word, low nibble first) and scales/biases
 // [N, K/64] in the activation dtype (bf16).
 //
-// Three kernels: the exact-product kernel below (M <= 512), the decode kernel
-// for M <= 64 with K a multiple of 512 and the hi/lo-plane kernel for M > 512
-// (further down).
+// Four kernels: the decode kernel for M <= 64 with K a multiple of 512
+// (further down), the tiles of qgemm_tile.hip for more rows of such K, and
+// for other K (or operands those do not take) the exact-product kernel below
+// (M <= 512) and the hi/lo-plane kernel (M > 512).
 //
 // Exact products, one group at a time. A code q enters the matrix core as
 // the bf16 number 128 + q (two bit operations per pair of codes), x as
@@ -1516,6 +1517,8 @@ void qgemm_launch(const QgemmArgs& a, hipStream_t s) {
   const unsigned gx = (unsigned)((a.N + kQgBN - 1) / kQgBN);
   if (a.M <= 64 && decode_fits(a)) {
     decode_launch(a, s);
+  } else if (qgemm_tile_fits(a)) {
+    qgemm_tile_launch(a, s);
   } else if (a.M <= 512) {
     HGK_LAUNCH(qgemm_kernel<64>, dim3(gx, (unsigned)((a.M + 63) / 64)), dim3(256), 0, s, a);
   } else {

@@ -65,6 +65,29 @@ def test_decode_wide_projection(dev, M, N):
     _check(got, ref, O.BF16, f"decode M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K,ys", [(65, 64, 512, 0), (129, 200, 1024, 0), (301, 1001, 512, 0),
+                                      (300, 512, 12288, 8), (1024, 2048, 512, 0),
+                                      (640, 8200, 512, 3), (700, 12288, 512, 0),
+                                      (2050, 6150, 1024, 0), (4100, 12288, 512, 0)],
+                         ids=["first-rows", "ragged", "odd-N", "long-K", "full-chip",
+                              "odd-y-stride", "64x128", "128x128", "256x256"])
+def test_tile_sizes(dev, M, N, K, ys):
+    """Rows past the decode kernel: every tile size the launch chooses from,
+    ragged rows and columns, y rows that are not 16-byte aligned. Large shapes
+    are checked on rows and columns around the tile edges. |y - ref| <= 1 bf16
+    ulp, as for every contraction: all products are exact, the sums f32."""
+    x, w, s, b = _case(3801 + M + N, M, N, K)
+    buf = torch.zeros((M, N + ys), dtype=torch.bfloat16, device=dev)
+    H.quantized_matmul(to_dev(x, O.BF16, dev), words_dev(w, dev), to_dev(s, O.BF16, dev),
+                       to_dev(b, O.BF16, dev), out=buf[:, :N])
+    got = to_host(buf)
+    assert (O.to_f32(got[:, N:], O.BF16) == 0).all()
+    rows = np.unique(np.clip(np.r_[0:3, 62:66, 126:130, 254:258, M // 2, M - 70, M - 3:M], 0, M - 1))
+    cols = np.unique(np.clip(np.r_[0:70, 120:140, 250:260, N // 2:N // 2 + 8, N - 140:N], 0, N - 1))
+    ref = O.quantized_matmul(x[rows], O.BF16, w[cols], s[cols], b[cols], O.BF16)
+    _check(got[:, :N][np.ix_(rows, cols)], ref, O.BF16, f"M={M} N={N} K={K}")
+
+
 def test_qwen3_next_prefill_projection(dev):
     """A 2048-token prefill through a 2048 -> 4096 projection (the attention
     q projection's shape class)."""
