@@ -52,7 +52,17 @@ void gather_grouped_launch(const GatherArgs& a, hipStream_t s);
 // bi2: up, same shapes); false where the fused kernel does not apply.
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s);
 
-// Rows of x at or above which the MFMA kernel runs (below: one GEMV per row).
+// Rows of x at or above which the MFMA kernels run for every K. Below, they
+// run where the decode kernel takes the call (K a multiple of 512, scales and
+// biases 4-byte aligned): it reads each weight once for all rows, while the
+// GEMV kernels read them once per row (and, for K other than 512, 1024, 2048
+// and 4096, one element at a time: 80 us at 1 x 4096 x 12288 against 20).
+// us per call, GEMV / decode kernel:
+//   N x K           1 row         4 rows        15 rows
+//   12288 x 4096    12.8 / 11.8   23.6 / 12.3   59.7 / 13.7
+//   12288 x 2048    7.5 / 6.9     11.2 / 6.9    25.9 / 7.3
+//   2048 x 2048     5.4 / 4.6     5.5 / 4.9     7.5 / 5.5
+//   512 x 2048      4.7 / 4.3     4.8 / 4.6     5.0 / 5.2
 constexpr int64_t kQgemmMinRows = 16;
 
 // bf16 activations and scales, group 64, 4 bits, x 16-byte aligned with a
@@ -60,6 +70,7 @@ constexpr int64_t kQgemmMinRows = 16;
 bool qgemm_supported(int dtype, int sdt, int group_size, int bits, const void* x, int64_t xs,
                      const void* w, int64_t k);
 void qgemm_launch(const QgemmArgs& a, hipStream_t s);
+bool qgemm_few_rows_fits(const QgemmArgs& a);
 
 // Many rows (qgemm_tile.hip): K a multiple of 512, w 16-byte and scales and
 // biases 4-byte aligned, a block's rows and columns within 2 GiB.

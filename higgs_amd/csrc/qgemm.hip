@@ -1513,6 +1513,10 @@ bool qgemm_supported(int dtype, int sdt, int group_size, int bits, const void* x
          (reinterpret_cast<uintptr_t>(w) & 7) == 0 && ((k / 8) % 2) == 0;
 }
 
+bool qgemm_few_rows_fits(const QgemmArgs& a) {
+  return decode_fits(a) && ((reinterpret_cast<uintptr_t>(a.sc) | reinterpret_cast<uintptr_t>(a.bi)) & 3) == 0;
+}
+
 void qgemm_launch(const QgemmArgs& a, hipStream_t s) {
   const unsigned gx = (unsigned)((a.N + kQgBN - 1) / kQgBN);
   if (a.M <= 64 && decode_fits(a)) {

@@ -420,15 +420,16 @@ extern "C" int hgk_quantized_matmul(int dtype, const void* x, int64_t m, int64_t
     return fail(HGK_ERR_UNSUPPORTED, "%s: problem too large", fn);
   if (m == 0) return HGK_OK;
   const hipStream_t s = as_stream(stream);
-  if (m >= kQgemmMinRows &&
-      qgemm_supported(dtype, scales_dtype, group_size, bits, x, x_row_stride, w, k) &&
+  if (qgemm_supported(dtype, scales_dtype, group_size, bits, x, x_row_stride, w, k) &&
       (m + 127) / 128 <= 65535) {
     QgemmArgs g{};
     g.x = static_cast<const uint16_t*>(x); g.xs = x_row_stride; g.w = w;
     g.sc = static_cast<const uint16_t*>(scales); g.bi = static_cast<const uint16_t*>(biases);
     g.M = m; g.N = n; g.K = k; g.y = static_cast<uint16_t*>(y); g.ys = y_row_stride;
-    qgemm_launch(g, s);
-    return launch_status(fn);
+    if (m >= kQgemmMinRows || qgemm_few_rows_fits(g)) {
+      qgemm_launch(g, s);
+      return launch_status(fn);
+    }
   }
   if (m * n >= ((int64_t)1 << 32))
     return fail(HGK_ERR_UNSUPPORTED, "%s: M=%lld x N=%lld too large for the per-row path", fn,

@@ -392,8 +392,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
     """quantized_matmul(x, w, scales, biases, transpose, group_size, bits) as
     QLinear::forward calls it (qwen3_next.rs:174-221): x [..., K], w [N,
     K*bits/32] packed 32-bit words, scales/biases [N, K/group_size]. Returns
-    y [..., N] in x's dtype. M >= 16 rows in bf16 with group 64 run on the
-    matrix cores; fewer rows, f16 or other groups run one GEMV per row."""
+    y [..., N] in x's dtype. bf16 with group 64 runs on the matrix cores (fewer
+    than 16 rows: where K is a multiple of 512); f16, other groups and the rest
+    run one GEMV per row."""
     if not transpose:
         raise HgkError(2, "quantized_matmul: only transpose=True (weights stored [N, K]) is implemented")
     if w.dim() != 2 or scales.dim() != 2 or scales.shape != biases.shape:

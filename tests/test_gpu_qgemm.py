@@ -108,6 +108,17 @@ def test_few_rows_take_the_gemv_path(dev, M):
     _check(got, ref, O.BF16, f"M={M}")
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 17, 512), (1, 4096, 3584), (2, 1000, 2048), (1, 512, 12288),
+                                   (15, 64, 8192), (7, 12289, 512)])
+def test_few_rows_on_the_decode_kernel(dev, M, N, K):
+    """1 to 15 rows with K a multiple of 512: column tiles that are partly
+    filled, K beyond the GEMV's list, few and many column tiles."""
+    x, w, s, b = _case(3901 + M + N, M, N, K)
+    got = _run(dev, x, w, s, b, O.BF16)
+    ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
+    _check(got, ref, O.BF16, f"M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("dt,group", [(O.F16, 64), (O.BF16, 32), (O.BF16, 128)])
 def test_other_dtypes_and_groups(dev, dt, group):
     x, w, s, b = _case(3300 + group, 40, 256, 1024, group=group, dt=dt)
