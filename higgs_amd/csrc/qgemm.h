@@ -42,8 +42,9 @@ struct GatherArgs {
 constexpr int64_t kGatherMinPairsPerExpert = 16;
 
 // bf16, group 64, 4 bits, x 16-byte aligned rows, w 16-byte aligned, K % 64,
-// the expert ids 16-byte aligned and a multiple of 4 (read 4 at a time: a
-// partly out-of-range 16-byte buffer load is not relied on) and under 2 GiB.
+// the expert ids 16-byte aligned (read 4 at a time, the last up to 3 one by
+// one: a partly out-of-range 16-byte buffer load is not relied on) and under
+// 2 GiB.
 bool gather_grouped_supported(int dtype, int sdt, int group_size, int bits, const void* x,
                               int64_t xs, const void* w, int64_t k, const void* experts,
                               int64_t pairs);

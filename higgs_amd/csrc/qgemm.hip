@@ -755,7 +755,8 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
   const int lane = tid & 63;
   // raw ids equal to e (and, for int32 ids, to e - E, which wraps to e)
   const uint32_t e1 = (uint32_t)e, e2 = a.experts_i32 ? (uint32_t)(e - a.E) : (uint32_t)e;
-  const uint32_t pairs = (uint32_t)a.pairs;
+  // ids of the last, partly filled 16 bytes (up to 3) are read one by one
+  const uint32_t pairs = (uint32_t)a.pairs & ~3u, tail = (uint32_t)a.pairs & 3u;
   auto load_round = [&](uint32_t (&r)[RND], int64_t base) {
     const bool live = base < a.pairs;
 #pragma unroll
@@ -790,6 +791,12 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
           base += __popcll(bal[i]);
         }
       }
+    }
+    // the round that reaches the last ids has at most kGaRoundIds - 4 others
+    if (tail && scan <= pairs && pairs < scan + kGaRoundIds && tid < 64) {  // uniform per wave
+      const bool in = lane < (int)tail;
+      const uint32_t id = reinterpret_cast<const uint32_t*>(a.experts)[pairs + (in ? lane : 0)];
+      if (in && (id == e1 || id == e2)) list[atomicAdd(cnt, 1)] = (int32_t)(pairs + lane);
     }
     scan += kGaRoundIds;
     __syncthreads();
@@ -851,7 +858,7 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   // the last pair read zeros and are never listed)
   static_assert(RND % 4 == 0, "whole 16-byte id loads");
   const __amdgpu_buffer_rsrc_t rid = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<void*>(a.experts), (short)0, (int)(a.pairs * 4), 0x00020000);
+      const_cast<void*>(a.experts), (short)0, (int)(a.pairs / 4 * 16), 0x00020000);
   int64_t scan = 0;
   while (scan < a.pairs) {
     // ---- fill the list from `scan` (stop before overflow)
@@ -1032,7 +1039,7 @@ constexpr int kXpBN = 64 * kXpWaves;  // columns per block pass
 // up waves leave their bf16 results in LDS and the gate waves write
 // swiglu(gate, up), rounded as the reference's three calls round it.
 template <int RT, bool SW>
-__global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a) {
+__global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t part) {
   constexpr int BM = 16 * RT, NT = 4;
   constexpr int BNO = SW ? kXpBN / 2 : kXpBN;  // output columns per pass
   constexpr int XP = (BM * 8 + kXpT - 1) / kXpT;  // 16-byte x pieces per thread per group
@@ -1053,10 +1060,15 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a) {
   const int nt0 = (int)blockIdx.x * tpg, nt1 = nt0 + tpg < ntiles ? nt0 + tpg : ntiles;
   const int G = (int)(a.K / 64);
 
+  // this block's part of the pairs (one part unless there are few experts)
+  int64_t scan = (int64_t)blockIdx.z * part;
+  const __amdgpu_buffer_rsrc_t rid = buf_rsrc(a.experts, (uint32_t)(a.pairs / 4 * 16));
+  a.pairs = scan + part < a.pairs ? scan + part : a.pairs;
+
   if (e == a.E) {
     // pairs whose expert is out of range: zero rows (this block's columns)
     const int64_t c0 = (int64_t)nt0 * BNO, c1 = (int64_t)nt1 * BNO < a.N ? (int64_t)nt1 * BNO : a.N;
-    for (int64_t p0 = 0; p0 < a.pairs; p0 += kXpT) {
+    for (int64_t p0 = scan; p0 < a.pairs; p0 += kXpT) {
       const int64_t p = p0 + tid;
       const int64_t ep = p < a.pairs ? ga_expert(a, p) : 0;
       if (p < a.pairs && (ep < 0 || ep >= a.E))
@@ -1066,8 +1078,6 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a) {
   }
 
   static_assert(RND % 4 == 0, "whole 16-byte id loads");
-  const __amdgpu_buffer_rsrc_t rid = buf_rsrc(a.experts, (uint32_t)(a.pairs * 4));
-
   const uint32_t xbytes = (uint32_t)(((a.xrows - 1) * a.xs + a.K) * 2);
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(a.x, xbytes);
   // the up waves (SW, waves 4-7: also the threads staging the up columns'
@@ -1149,7 +1159,6 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a) {
   };
   const X4Masks xm = x4_masks();
 
-  int64_t scan = 0;
   while (scan < a.pairs) {
     // ---- list this expert's pairs from `scan` (stop before overflow)
     const int rows = ga_list_phase<RND>(a, rid, e, scan, tid, &cnt, list);
@@ -1385,7 +1394,7 @@ bool gather_grouped_supported(int dtype, int sdt, int group_size, int bits, cons
   return dtype == DT_BF16 && sdt == DT_BF16 && group_size == 64 && bits == 4 && k % 64 == 0 &&
          (reinterpret_cast<uintptr_t>(x) & 15) == 0 && xs % 8 == 0 &&
          (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
-         (reinterpret_cast<uintptr_t>(experts) & 15) == 0 && pairs % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(experts) & 15) == 0 &&
          pairs * 4 < ((int64_t)1 << 31);
 }
 
@@ -1404,38 +1413,45 @@ bool gather_xp_fits(const GatherArgs& a) {
          a.E * a.N * (a.K / 64) * 2 < lim;
 }
 
+// The grid: column tiles split over about 1024 blocks in all (each block lists
+// its expert's pairs once for its tiles: at 512 experts and 4 tiles, the
+// 2048-column down projection, 1 block per expert measured 224-225 us against
+// 232 with 2 and 265 with 4), and, where that leaves fewer blocks than CUs
+// (few experts), the pairs split in parts that still fill a pass of rows per
+// expert: 4096 tokens x 8 of 64 experts, 2048 -> 512: fused gate + up 408 ->
+// 264 us, gate 355 -> 126 (128 and 64 blocks before, 512 and 320 now). With a
+// block per CU already, parts gained nothing (8 of 128 experts, 2048 -> 1024:
+// gate 224 us, 259 in two parts): each part reads the weights again.
+template <bool SW>
 void gather_xp_launch(const GatherArgs& a, hipStream_t s) {
-  const int64_t ntiles = (a.N + kXpBN - 1) / kXpBN;
-  // column tiles split over about 1024 blocks in all: each block lists its
-  // expert's pairs once for its tiles. At 512 experts and 4 tiles (the
-  // 2048-column down projection) 1 block per expert measured 224-225 us,
-  // against 232 with 2 and 265 with 4 (with 96-row passes 2 had been best:
-  // 244 against 261).
+  constexpr int BNO = SW ? kXpBN / 2 : kXpBN;
+  const int64_t ntiles = (a.N + BNO - 1) / BNO;
   int64_t gx = 1024 / (a.E + 1);
   gx = gx < 1 ? 1 : (gx > ntiles ? ntiles : gx);
   const int64_t tpg = (ntiles + gx - 1) / gx;
   gx = (ntiles + tpg - 1) / tpg;
-  const dim3 grid((unsigned)gx, (unsigned)(a.E + 1));
-  HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, false>), grid, dim3(kXpT), 0, s, a);
+  int64_t gz = 1;
+  if (a.E * gx < kCUs) {
+    const int64_t fill = 2 * kCUs / (a.E * gx), full = a.pairs / (a.E * 16 * HGK_XP_RT);
+    gz = fill < full ? fill : full;
+    gz = gz < 1 ? 1 : gz;
+  }
+  const int64_t part = ((a.pairs + gz - 1) / gz + 3) / 4 * 4;
+  const dim3 grid((unsigned)gx, (unsigned)(a.E + 1), (unsigned)((a.pairs + part - 1) / part));
+  HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW>), grid, dim3(kXpT), 0, s, a, part);
 }
 
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s) {
   if (!HGK_GATHER_XP || !gather_xp_fits(a) || !a.w2 || !a.sc2 || !a.bi2 ||
       (reinterpret_cast<uintptr_t>(a.w2) & 15) != 0)
     return false;
-  const int64_t ntiles = (a.N + kXpBN / 2 - 1) / (kXpBN / 2);
-  int64_t gx = 1024 / (a.E + 1);
-  gx = gx < 1 ? 1 : (gx > ntiles ? ntiles : gx);
-  const int64_t tpg = (ntiles + gx - 1) / gx;
-  gx = (ntiles + tpg - 1) / tpg;
-  const dim3 grid((unsigned)gx, (unsigned)(a.E + 1));
-  HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, true>), grid, dim3(kXpT), 0, s, a);
+  gather_xp_launch<true>(a, s);
   return true;
 }
 
 void gather_grouped_launch(const GatherArgs& a, hipStream_t s) {
   if (HGK_GATHER_XP && gather_xp_fits(a)) {
-    gather_xp_launch(a, s);
+    gather_xp_launch<false>(a, s);
     return;
   }
   // column tiles are split over as many blocks as keep about 1024 blocks in

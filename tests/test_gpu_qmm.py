@@ -278,6 +278,25 @@ def test_grouped_size_with_unaligned_pair_count(dev):
     _check(got[-2:], ref[-2:], O.BF16, "last pairs")
 
 
+@pytest.mark.parametrize("P,K", [(4097, 512), (8191, 512), (2 * 6146, 512), (4099, 576)],
+                         ids=["one-past-a-round", "three", "two-long-lists", "other-K"])
+def test_grouped_last_pairs_and_parts(dev, P, K):
+    """Pair counts that end 1, 2 or 3 past a 16-byte read of the ids, with few
+    experts (their pairs are split over several blocks where K is a multiple
+    of 512), one of them taking half of all pairs, and ids out of range."""
+    R, E, N = 400, 4, 200
+    x, w, s, b, ex = _case(2481 + P, P, R, E, N, K)
+    ex[::2] = 1
+    ex[[5, P - 1]] = [E, -E - 1]
+    ex[P - 2] = -2
+    lhs = ((np.arange(P) * 7) % R).astype(np.int32)
+    got = _run(dev, x, w, s, b, ex, O.BF16, lhs=lhs)
+    assert not got[[5, P - 1]].any()
+    rows = np.unique(np.r_[0:5, 6:200, P // 2 - 70:P // 2 + 70, P - 300:P - 1])
+    ref = O.gather_qmm(x, O.BF16, w, s, b, O.BF16, np.where(ex < 0, ex + E, ex)[rows], lhs=lhs[rows])
+    _check(got[rows], ref, O.BF16, f"grouped P={P} K={K}")
+
+
 # ------------------------------------------------------------------ fused gate/up/SwiGLU
 def _fused_case(key, T, top_k, E, N, K, group=64):
     P = T * top_k
