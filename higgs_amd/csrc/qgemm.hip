@@ -749,14 +749,15 @@ __device__ inline int64_t ga_row(const GatherArgs& a, int64_t p) {
 // prefill. The list order is free: every listed pair's output row is
 // computed on its own.
 // Contains barriers: every thread of the block calls it. Returns the count.
-template <int RND>
+// Without TAIL the pair count must be a multiple of 4.
+template <int RND, bool TAIL>
 __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t rid, int64_t e,
                                     int64_t& scan, int tid, int* cnt, int32_t* list) {
   const int lane = tid & 63;
   // raw ids equal to e (and, for int32 ids, to e - E, which wraps to e)
   const uint32_t e1 = (uint32_t)e, e2 = a.experts_i32 ? (uint32_t)(e - a.E) : (uint32_t)e;
   // ids of the last, partly filled 16 bytes (up to 3) are read one by one
-  const uint32_t pairs = (uint32_t)a.pairs & ~3u, tail = (uint32_t)a.pairs & 3u;
+  const uint32_t tail = TAIL ? (uint32_t)a.pairs & 3u : 0u, pairs = (uint32_t)a.pairs - tail;
   auto load_round = [&](uint32_t (&r)[RND], int64_t base) {
     const bool live = base < a.pairs;
 #pragma unroll
@@ -792,12 +793,6 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
         }
       }
     }
-    // the round that reaches the last ids has at most kGaRoundIds - 4 others
-    if (tail && scan <= pairs && pairs < scan + kGaRoundIds && tid < 64) {  // uniform per wave
-      const bool in = lane < (int)tail;
-      const uint32_t id = reinterpret_cast<const uint32_t*>(a.experts)[pairs + (in ? lane : 0)];
-      if (in && (id == e1 || id == e2)) list[atomicAdd(cnt, 1)] = (int32_t)(pairs + lane);
-    }
     scan += kGaRoundIds;
     __syncthreads();
   };
@@ -814,6 +809,13 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
     load_round(ra, scan + kGaRoundIds);
     round(rb);
   }
+  if (tail && scan >= a.pairs) {  // uniform; the list has room for 3 more
+    if (tid < (int)tail) {
+      const uint32_t id = reinterpret_cast<const uint32_t*>(a.experts)[pairs + tid];
+      if (id == e1 || id == e2) list[atomicAdd(cnt, 1)] = (int32_t)(pairs + tid);
+    }
+    __syncthreads();
+  }
   return *cnt;
 }
 
@@ -827,7 +829,7 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   __shared__ __align__(16) uint16_t xs[2][kGaBM][kQgPitch];
   __shared__ __align__(16) uint16_t wh[2][kHlBN][kQgPitch];
   __shared__ __align__(16) uint16_t wl[2][kHlBN][kQgPitch];
-  __shared__ int32_t list[kGaCap];
+  __shared__ int32_t list[kGaCap + 4];
   __shared__ int32_t cnt;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -862,7 +864,7 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   int64_t scan = 0;
   while (scan < a.pairs) {
     // ---- fill the list from `scan` (stop before overflow)
-    const int rows = ga_list_phase<RND>(a, rid, e, scan, tid, &cnt, list);
+    const int rows = ga_list_phase<RND, true>(a, rid, e, scan, tid, &cnt, list);
 
     // ---- the listed pairs, kGaBM at a time, for each of this block's column tiles
     for (int nt = nt0; nt < nt1; ++nt)
@@ -1038,7 +1040,11 @@ constexpr int kXpBN = 64 * kXpWaves;  // columns per block pass
 // and waves 4-7 the up projection of the same 256 columns; after a pass the
 // up waves leave their bf16 results in LDS and the gate waves write
 // swiglu(gate, up), rounded as the reference's three calls round it.
-template <int RT, bool SW>
+// GEN: any pair count, and the pairs split over gridDim.z blocks, `part` pairs
+// each. Its own form: the usual one (a multiple of 4, one part) keeps its
+// registers (with the last ids' code in it, it spilled 20 bytes and ran 1.5 %
+// slower).
+template <int RT, bool SW, bool GEN>
 __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t part) {
   constexpr int BM = 16 * RT, NT = 4;
   constexpr int BNO = SW ? kXpBN / 2 : kXpBN;  // output columns per pass
@@ -1048,7 +1054,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
   __shared__ float sxs[8][BM];              // row sums, ring of 8 groups
   // scales and biases of 8 groups per column (double-buffered per 8 groups)
   __shared__ __align__(16) u32x4 ssb[2][kXpBN], bsb[2][kXpBN];
-  __shared__ int32_t list[kGaCap];
+  __shared__ int32_t list[kGaCap + 4];
   __shared__ int32_t cnt;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1060,10 +1066,13 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
   const int nt0 = (int)blockIdx.x * tpg, nt1 = nt0 + tpg < ntiles ? nt0 + tpg : ntiles;
   const int G = (int)(a.K / 64);
 
-  // this block's part of the pairs (one part unless there are few experts)
-  int64_t scan = (int64_t)blockIdx.z * part;
+  // this block's part of the pairs
+  int64_t scan = 0;
   const __amdgpu_buffer_rsrc_t rid = buf_rsrc(a.experts, (uint32_t)(a.pairs / 4 * 16));
-  a.pairs = scan + part < a.pairs ? scan + part : a.pairs;
+  if constexpr (GEN) {
+    scan = (int64_t)blockIdx.z * part;
+    a.pairs = scan + part < a.pairs ? scan + part : a.pairs;
+  }
 
   if (e == a.E) {
     // pairs whose expert is out of range: zero rows (this block's columns)
@@ -1161,7 +1170,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
 
   while (scan < a.pairs) {
     // ---- list this expert's pairs from `scan` (stop before overflow)
-    const int rows = ga_list_phase<RND>(a, rid, e, scan, tid, &cnt, list);
+    const int rows = ga_list_phase<RND, GEN && !SW>(a, rid, e, scan, tid, &cnt, list);
 
     for (int nt = nt0; nt < nt1; ++nt)
     for (int t0 = 0; t0 < rows; t0 += BM) {
@@ -1438,7 +1447,10 @@ void gather_xp_launch(const GatherArgs& a, hipStream_t s) {
   }
   const int64_t part = ((a.pairs + gz - 1) / gz + 3) / 4 * 4;
   const dim3 grid((unsigned)gx, (unsigned)(a.E + 1), (unsigned)((a.pairs + part - 1) / part));
-  HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW>), grid, dim3(kXpT), 0, s, a, part);
+  if (grid.z > 1 || a.pairs % 4 != 0)
+    HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, true>), grid, dim3(kXpT), 0, s, a, part);
+  else
+    HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, false>), grid, dim3(kXpT), 0, s, a, part);
 }
 
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s) {
