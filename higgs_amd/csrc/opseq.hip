@@ -14,13 +14,23 @@
 // workgroup barriers between ops; no workgroup ever waits on another, so the
 // grid needs no co-residency and no wait can hang.
 //
-// Each op waits for the previous op's stores to complete before any thread of
-// the workgroup issues its first load (a wait on every outstanding memory
-// operation, then the workgroup barrier), as the next op of a real layer
-// would need them: the launch's time is the latency of the dependent chain,
-// not the throughput of independent ops. Every consumer of an op's output
-// inside the launch is the same workgroup, so workgroup-scope ordering is all
-// the data needs; other consumers see it after the launch.
+// Most of those ops do not depend on each other: of the 192 ops of a 48-layer
+// Qwen3-Next step, 96 form the residual chain and 96 read nothing that the
+// list writes. Upload therefore sorts the ops into chains (ops that share a
+// buffer, one of them writing it, for the same token stay in one chain, in
+// list order), and a token gets kChains workgroups, one per chain. Within a
+// chain an op waits for earlier stores (a wait on every outstanding memory
+// operation, then the workgroup barrier) only where it touches what an op
+// since the last wait wrote, and a run of residual adds + norms over the same
+// rows carries h in registers, with the next residual and weight loaded
+// beside the current sum. 64 tokens x 48 layers: 466 us with every op in one
+// workgroup, waiting; 159 with chains.
+// Every consumer of an op's output inside the launch is the same workgroup,
+// so workgroup-scope ordering is all the data needs; other consumers see it
+// after the launch. Buffers that only meet for some later token (views with
+// different token strides) bound the token count up to which the chains hold
+// (`safe`); a run over more tokens walks the whole list in one workgroup per
+// token, waiting after every op.
 //
 // Each op's arithmetic is the standalone kernel's (norm.hip, rope.hip,
 // glu.hip) for 16-bit activations and weights of the same type: results are
@@ -42,13 +52,17 @@ namespace hgk {
 constexpr uint32_t kOpListMagic = 0x6f70736bu;  // "opsk"
 constexpr int kOpMaxHalf = 256;                 // rotated dims / 2
 constexpr int kOpThreads = 1024;
+constexpr int kChains = 8;                      // workgroups per token
 
 // One op as the kernel reads it (written by the host from an hgk_op).
 struct alignas(16) DevOp {
   int32_t kind, act, rows, n;
   int32_t k_rows, dims, half, lpr;      // rope: k heads, rotated dims, dims / 2, lanes per row
-  int32_t g, same_table, pad0, pad3;    // norms: lanes per row; rope: the cos/sin table of
-                                        // the previous rope op serves (same positions, freqs)
+  int32_t g, same_table;                // norms: lanes per row; rope: the cos/sin table of the
+                                        // previous rope op (bit 0: of the list, bit 1: of the
+                                        // chain) serves (same positions, frequencies)
+  int32_t next;                         // the chain's next op (INT32_MAX: none)
+  int32_t flags;                        // kOpWait, kOpCarry
   float eps, inv_n, scale, pad1;
   int64_t zg, zgs;                      // gated: z rows per group, group stride
   const void* x; int64_t x_tok, x_row;  // x / gate / q
@@ -57,7 +71,8 @@ struct alignas(16) DevOp {
   void* y; int64_t y_tok, y_row;        // y / out / q out
   void* h; int64_t h_tok, h_row;        // residual out / k out
   const int32_t* offsets;
-  int32_t offset, pad2;
+  int32_t offset;
+  int32_t first;                        // in op c: the first op of chain c (INT32_MAX: none)
   float inv_freq[kOpMaxHalf];
 };
 
@@ -65,7 +80,7 @@ struct alignas(16) DevOpList {
   uint32_t magic;
   int32_t dtype;
   int32_t count;
-  int32_t pad;
+  int32_t safe;         // tokens up to which the chains are independent
   DevOp ops[1];  // count entries
 };
 
@@ -73,13 +88,12 @@ constexpr int64_t op_list_bytes(int n) {
   return (int64_t)sizeof(DevOpList) + (int64_t)(n - 1) * (int64_t)sizeof(DevOp);
 }
 
+// kOpWait: in its chain, the op waits for the stores before it. kOpCarry: its x
+// is the h of the chain's previous op, an add + norm over the same rows (one
+// 16-byte unit per thread), so it is taken from registers.
+enum { kOpWait = 1, kOpCarry = 2 };
 enum { kOpRms = 0, kOpAddRms = 1, kOpGated = 2, kOpRope = 3, kOpGlu = 4 };
 
-// Whether an op waits for its stores to complete before the next op starts
-// (1), or only orders them before the next op's loads through the barrier (0).
-#ifndef HGK_OPSEQ_STORE_WAIT
-#define HGK_OPSEQ_STORE_WAIT 1
-#endif
 // Whether each op brings the next op's descriptor into the scalar cache.
 #ifndef HGK_OPSEQ_PREFETCH
 #define HGK_OPSEQ_PREFETCH 1
@@ -88,7 +102,7 @@ enum { kOpRms = 0, kOpAddRms = 1, kOpGated = 2, kOpRope = 3, kOpGlu = 4 };
 // Every store of this op has completed before any thread of the workgroup
 // issues the next op's loads.
 __device__ inline void op_boundary() {
-  if (HGK_OPSEQ_STORE_WAIT) __builtin_amdgcn_s_waitcnt(0);  // all counters: loads, stores, LDS
+  __builtin_amdgcn_s_waitcnt(0);  // all counters: loads, stores, LDS
   __syncthreads();
 }
 
@@ -185,6 +199,97 @@ __device__ void op_norm(const DevOp& op, int64_t t, double* part) {
   }
 }
 
+// A run of add + norm ops of one chain over the same rows (at most one row per
+// lane group): op i and the ops after it that take their x from its h in
+// registers. The next op's r and weight are loaded before the current sum, and
+// the sum's LDS slots alternate, so an op costs one workgroup barrier.
+// Returns the last op's index.
+template <class X, int G>
+__device__ int op_add_run(const DevOpList* list, int i, int n_ops, int64_t t, double (*part)[kOpThreads / 64]) {
+  constexpr int V = Vec<X>::N;
+  const int row = threadIdx.x / G, j = threadIdx.x % G;
+  const DevOp* op = &list->ops[i];
+  const int nch = op->n / V;
+  const bool own = row < op->rows && j < nch;
+  const int rr = row < op->rows ? row : op->rows - 1, chc = j < nch ? j : nch - 1;
+  auto at = [&](const void* p, int64_t tok, int64_t rs) {
+    return reinterpret_cast<const char*>(p) + (t * tok + (int64_t)rr * rs + (int64_t)chc * V) * X::kBytes;
+  };
+  auto weight = [&](const DevOp* o) {
+    return o->w ? ld16<X>(o->w, (int64_t)chc * V) : u32x4{0u, 0u, 0u, 0u};
+  };
+  u32x4 xr = ld16<X>(at(op->x, op->x_tok, op->x_row), 0);
+  u32x4 r = ld16<X>(at(op->r, op->r_tok, op->r_row), 0);
+  u32x4 w = weight(op);
+  for (int par = 0;; par ^= 1) {
+    const int nx = op->next;
+    const DevOp* const no = &list->ops[nx < n_ops ? nx : i];
+    const bool more = nx < n_ops && (no->flags & kOpCarry);  // uniform
+    u32x4 nr = r, nw = w;
+    if (more) {
+      nr = ld16<X>(at(no->r, no->r_tok, no->r_row), 0);
+      nw = weight(no);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      xr[k] = X::pack(X::lo(xr[k]) + X::lo(r[k]), X::hi(xr[k]) + X::hi(r[k]));
+    if (op->h && own) *reinterpret_cast<u32x4*>(const_cast<char*>(at(op->h, op->h_tok, op->h_row))) = xr;
+    double ss = 0.0;
+    if (j < nch) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const double d = (double)elem<X>(xr, e);
+        ss = __builtin_fma(d, d, ss);
+      }
+    }
+    if constexpr (G <= 64) {
+      ss = group_sum<G>(ss);
+    } else {
+      ss = group_sum<64>(ss);
+      const int wave = threadIdx.x >> 6;
+      if ((threadIdx.x & 63) == 0) part[par][wave] = ss;
+      __syncthreads();
+      constexpr int WPG = G / 64;
+      ss = 0.0;
+#pragma unroll
+      for (int k = 0; k < WPG; ++k) ss += part[par][wave / WPG * WPG + k];
+    }
+    const float rs = rms_scale(ss, op->inv_n, op->eps);
+    if (own) {
+      float o[V];
+#pragma unroll
+      for (int e = 0; e < V; e += 2) {
+        float n0 = elem<X>(xr, e) * rs, n1 = elem<X>(xr, e + 1) * rs;
+        round2<X>(n0, n1);
+        o[e] = n0 * (op->w ? elem<X>(w, e) : 1.0f);
+        o[e + 1] = n1 * (op->w ? elem<X>(w, e + 1) : 1.0f);
+      }
+      store_elems<X, V, false>(const_cast<char*>(at(op->y, op->y_tok, op->y_row)), 0, o);
+    }
+    if (!more) return i;
+    op = no;
+    i = nx;
+    r = nr;
+    w = nw;
+  }
+}
+
+template <class X>
+__device__ int add_run_dispatch(const DevOpList* list, int i, int n_ops, int64_t t,
+                                double (*part)[kOpThreads / 64]) {
+  switch (list->ops[i].g) {
+    case 4: return op_add_run<X, 4>(list, i, n_ops, t, part);
+    case 8: return op_add_run<X, 8>(list, i, n_ops, t, part);
+    case 16: return op_add_run<X, 16>(list, i, n_ops, t, part);
+    case 32: return op_add_run<X, 32>(list, i, n_ops, t, part);
+    case 64: return op_add_run<X, 64>(list, i, n_ops, t, part);
+    case 128: return op_add_run<X, 128>(list, i, n_ops, t, part);
+    case 256: return op_add_run<X, 256>(list, i, n_ops, t, part);
+    case 512: return op_add_run<X, 512>(list, i, n_ops, t, part);
+    default: return op_add_run<X, 1024>(list, i, n_ops, t, part);
+  }
+}
+
 // q/k RMSNorm (where a weight is given) + RoPE of the token's q and k heads:
 // rope_kernel's two-chunk layout (lane j < R holds the rotation pair j, j + R;
 // the others hold two pass-through chunks), LPR lanes per head row, every
@@ -192,7 +297,7 @@ __device__ void op_norm(const DevOp& op, int64_t t, double* part) {
 // token's position from f64 sincos, rounded to X) lives in LDS; an op whose
 // positions and frequencies are those of the previous rope op reuses it.
 template <class X, int LPR>
-__device__ void op_rope(const DevOp& op, int64_t t, float* cs, float* sn) {
+__device__ void op_rope(const DevOp& op, int64_t t, bool same_table, float* cs, float* sn) {
   constexpr int V = Vec<X>::N;
   constexpr int P = kOpThreads / LPR;
   const int R = op.dims / (2 * V);
@@ -216,7 +321,7 @@ __device__ void op_rope(const DevOp& op, int64_t t, float* cs, float* sn) {
     const u32x4 d0 = ld16<X>(xp, (int64_t)c0 * V), d1 = ld16<X>(xp, (int64_t)c1 * V);
     const u32x4 wa = has ? ld16<X>(nw, (int64_t)c0 * V) : u32x4{0u, 0u, 0u, 0u};
     const u32x4 wb = has ? ld16<X>(nw, (int64_t)c1 * V) : u32x4{0u, 0u, 0u, 0u};
-    if (pass == 0 && !op.same_table) {  // built while the loads are in flight
+    if (pass == 0 && !same_table) {  // built while the loads are in flight
       const int32_t off = op.offsets ? op.offsets[t] : op.offset;
       const float pos = (0.0f + (float)off) * op.scale;
       for (int i = threadIdx.x; i < op.half; i += kOpThreads) {
@@ -328,41 +433,60 @@ __device__ void norm_dispatch(const DevOp& op, int64_t t, double* part) {
 
 template <class X>
 __global__ __launch_bounds__(kOpThreads) void opseq_kernel(const DevOpList* __restrict__ list,
-                                                           int n_ops) {
+                                                           int n_ops, int tokens, int chained) {
   __shared__ float cs[kOpMaxHalf], sn[kOpMaxHalf];
-  __shared__ double part[kOpThreads / 64];
-  const int64_t t = blockIdx.x;
+  __shared__ double part[2][kOpThreads / 64];
+  // block = (chain, token), all tokens of chain 0 (the longest) first
+  const int chain = blockIdx.x / (unsigned)tokens;
+  const int64_t t = blockIdx.x - (unsigned)chain * (unsigned)tokens;
   // a list that hgk_op_list_upload did not write for this dtype and length
   // is not walked (no pointer in it is trusted)
   if (list->magic != kOpListMagic || list->dtype != X::kCode || list->count < n_ops) return;
-  for (int i = 0; i < n_ops; ++i) {
+  const bool serial = !chained || tokens > list->safe;  // uniform over the grid
+  if (serial && chain > 0) return;
+  // the chain's first op (the header of op c holds chain c's)
+  int i = serial ? 0 : list->ops[chain < list->count ? chain : 0].first;
+  if (chain >= list->count) i = INT32_MAX;
+  while (i < n_ops) {
     const DevOp& op = list->ops[i];
+    if (!serial && (op.flags & kOpWait)) op_boundary();
+    int nx = serial ? i + 1 : op.next;
     uint32_t pf[4] = {0u, 0u, 0u, 0u};
-    if (HGK_OPSEQ_PREFETCH && i + 1 < n_ops) {
+    if (HGK_OPSEQ_PREFETCH && nx < n_ops) {
       // one dword of each 64-byte line of the next descriptor's fields
-      const uint32_t* nx = reinterpret_cast<const uint32_t*>(&list->ops[i + 1]);
-      pf[0] = nx[0]; pf[1] = nx[16]; pf[2] = nx[32]; pf[3] = nx[48];
+      const uint32_t* nd = reinterpret_cast<const uint32_t*>(&list->ops[nx]);
+      pf[0] = nd[0]; pf[1] = nd[16]; pf[2] = nd[32]; pf[3] = nd[48];
     }
     switch (op.kind) {
-      case kOpRms: norm_dispatch<X, kOpRms>(op, t, part); break;
-      case kOpAddRms: norm_dispatch<X, kOpAddRms>(op, t, part); break;
-      case kOpGated: norm_dispatch<X, kOpGated>(op, t, part); break;
-      case kOpRope:
-        switch (op.lpr) {
-          case 2: op_rope<X, 2>(op, t, cs, sn); break;
-          case 4: op_rope<X, 4>(op, t, cs, sn); break;
-          case 8: op_rope<X, 8>(op, t, cs, sn); break;
-          case 16: op_rope<X, 16>(op, t, cs, sn); break;
-          default: op_rope<X, 32>(op, t, cs, sn); break;
+      case kOpRms: norm_dispatch<X, kOpRms>(op, t, part[0]); break;
+      case kOpAddRms:
+        if (!serial && op.rows * op.g <= kOpThreads) {
+          nx = list->ops[add_run_dispatch<X>(list, i, n_ops, t, part)].next;
+        } else {
+          norm_dispatch<X, kOpAddRms>(op, t, part[0]);
         }
         break;
+      case kOpGated: norm_dispatch<X, kOpGated>(op, t, part[0]); break;
+      case kOpRope: {
+        const bool same = op.same_table & (serial ? 1 : 2);
+        switch (op.lpr) {
+          case 2: op_rope<X, 2>(op, t, same, cs, sn); break;
+          case 4: op_rope<X, 4>(op, t, same, cs, sn); break;
+          case 8: op_rope<X, 8>(op, t, same, cs, sn); break;
+          case 16: op_rope<X, 16>(op, t, same, cs, sn); break;
+          default: op_rope<X, 32>(op, t, same, cs, sn); break;
+        }
+        break;
+      }
       default:
         if (op.act == HGK_ACT_SILU) op_glu<X, HGK_ACT_SILU>(op, t);
         else op_glu<X, HGK_ACT_GELU_TANH>(op, t);
         break;
     }
     if (HGK_OPSEQ_PREFETCH) asm volatile("" ::"s"(pf[0]), "s"(pf[1]), "s"(pf[2]), "s"(pf[3]));
-    op_boundary();
+    if (serial) op_boundary();
+    else __syncthreads();  // the op's LDS is free
+    i = nx;
   }
 }
 
@@ -470,6 +594,149 @@ int translate(const hgk_op& s, int i, DevOp& d) {
   }
 }
 
+// Whether rope op d's cos/sin table is p's: same positions and frequencies.
+bool same_positions(const DevOp& p, const DevOp& d) {
+  return p.offsets == d.offsets && p.offset == d.offset && p.scale == d.scale && p.half == d.half &&
+         std::equal(d.inv_freq, d.inv_freq + d.half, p.inv_freq);
+}
+
+// The bytes an op reads or writes for token t: [lo + t tok, lo + t tok + span).
+struct Range {
+  int64_t lo, span, tok;
+  bool write;
+  int64_t row;  // row stride where one thread holds one 16-byte unit (add + norm), else -1
+};
+
+// The smallest t >= 0 for which a's and b's bytes of token t overlap.
+int64_t first_overlap(Range a, Range b) {
+  if (b.tok < a.tok) std::swap(a, b);
+  const int64_t d0 = b.lo - a.lo, dt = b.tok - a.tok;  // overlap: -b.span < d0 + t dt < a.span
+  if (d0 >= a.span) return INT64_MAX;
+  if (d0 > -b.span) return 0;
+  if (dt == 0) return INT64_MAX;
+  const int64_t t = (-b.span - d0) / dt + 1;  // the first t with d0 + t dt > -b.span
+  return d0 + t * dt < a.span ? t : INT64_MAX;
+}
+
+std::vector<Range> op_ranges(const DevOp& d) {
+  std::vector<Range> v;
+  const bool own = d.kind == kOpAddRms && d.rows * d.g <= kOpThreads;
+  auto add = [&](const void* p, int64_t tok, int64_t rows, int64_t row, bool write) {
+    if (p && rows > 0) v.push_back({(int64_t)(intptr_t)p, ((rows - 1) * row + d.n) * 2, tok * 2, write, own ? row : -1});
+  };
+  add(d.x, d.x_tok, d.rows, d.x_row, false);
+  add(d.y, d.y_tok, d.rows, d.y_row, true);
+  if (d.w) v.push_back({(int64_t)(intptr_t)d.w, d.n * 2, 0, false, -1});
+  if (d.kind == kOpAddRms || d.kind == kOpGlu) add(d.r, d.r_tok, d.rows, d.r_row, false);
+  if (d.kind == kOpAddRms) add(d.h, d.h_tok, d.rows, d.h_row, true);
+  if (d.kind == kOpGated) {
+    const int64_t groups = (d.rows + d.zg - 1) / d.zg, rows = std::min<int64_t>(d.rows, d.zg);
+    const int64_t far = (groups - 1) * d.zgs;  // may be negative
+    const int64_t lo = std::min<int64_t>(far, 0), hi = std::max<int64_t>(far, 0) + (rows - 1) * d.r_row + d.n;
+    v.push_back({(int64_t)(intptr_t)d.r + lo * 2, (hi - lo) * 2, d.r_tok * 2, false, -1});
+  }
+  if (d.kind == kOpRope) {
+    add(d.r, d.r_tok, d.k_rows, d.r_row, false);
+    add(d.h, d.h_tok, d.k_rows, d.h_row, true);
+    add(d.w2, 0, 1, 0, false);
+    if (d.offsets) v.push_back({(int64_t)(intptr_t)d.offsets, 4, 4, false, -1});
+  }
+  return v;
+}
+
+// Sort the list's ops into chains (see the top of the file).
+void make_chains(DevOpList* L) {
+  const int n = L->count;
+  std::vector<std::vector<Range>> rg(n);
+  for (int i = 0; i < n; ++i) rg[i] = op_ranges(L->ops[i]);
+  // The first token for which ops i < j conflict. carry: for j as a carried op
+  // (its x, range 0, is in registers), and where j writes exactly what i read or
+  // wrote, by the same threads (rows of the same shape), program order is enough.
+  auto conflict = [&](int i, int j, bool carry) {
+    const bool same = L->ops[i].rows == L->ops[j].rows && L->ops[i].n == L->ops[j].n;
+    int64_t t = INT64_MAX;
+    for (const Range& a : rg[i])
+      for (const Range& b : rg[j]) {
+        if (!a.write && !b.write) continue;
+        const bool layout = same && a.row >= 0 && a.row == b.row && a.lo == b.lo && a.tok == b.tok;
+        if (carry && layout && (b.write || (&b == &rg[j][0] && i == L->ops[j].next))) continue;
+        t = std::min(t, first_overlap(a, b));
+      }
+    return t;
+  };
+  std::vector<int> root(n), size(n, 1), chain(n);
+  for (int i = 0; i < n; ++i) root[i] = i;
+  auto find = [&](int i) {
+    while (root[i] != i) i = root[i] = root[root[i]];
+    return i;
+  };
+  int64_t safe = INT32_MAX;
+  for (int j = 0; j < n; ++j)
+    for (int i = 0; i < j; ++i) {
+      const int64_t t = conflict(i, j, false);
+      if (t > 0) {
+        safe = std::min(safe, t);
+      } else if (find(i) != find(j)) {
+        size[find(j)] += size[find(i)];
+        root[find(i)] = find(j);
+      }
+    }
+  // the largest group of dependent ops is chain 0; each other group goes to
+  // the chain with the fewest ops so far
+  int big = 0;
+  for (int i = 0; i < n; ++i)
+    if (size[find(i)] > size[find(big)]) big = i;
+  std::vector<int> of(n, -1);
+  int load[kChains] = {};
+  of[find(big)] = 0;
+  load[0] = size[find(big)];
+  for (int i = 0; i < n; ++i) {
+    int& c = of[find(i)];
+    if (c < 0) {
+      c = (int)(std::min_element(load, load + kChains) - load);
+      load[c] += size[find(i)];
+    }
+    chain[i] = c;
+  }
+  int last[kChains], since[kChains], rope[kChains];
+  for (int c = 0; c < kChains; ++c) {
+    last[c] = rope[c] = -1;
+    since[c] = 0;  // first op after the chain's last wait
+    if (c < n) L->ops[c].first = INT32_MAX;
+  }
+  for (int i = 0; i < n; ++i) {
+    DevOp& d = L->ops[i];
+    const int c = chain[i], p = last[c];
+    d.next = INT32_MAX;
+    d.flags = 0;
+    if (p < 0) {
+      L->ops[c].first = i;
+    } else {
+      DevOp& q = L->ops[p];
+      q.next = i;
+      const bool carry = d.kind == kOpAddRms && q.kind == kOpAddRms && q.h && d.x == q.h &&
+                         d.x_tok == q.h_tok && d.x_row == q.h_row && d.rows == q.rows && d.n == q.n &&
+                         d.rows * d.g <= kOpThreads;
+      // (d.next names the op whose h is carried until the chain's next op is known)
+      d.next = p;
+      bool wait = false;
+      for (int k = since[c]; k < i && !wait; ++k) wait = chain[k] == c && conflict(k, i, carry) == 0;
+      d.next = INT32_MAX;
+      if (carry && !wait) d.flags = kOpCarry;
+      if (wait) {
+        d.flags |= kOpWait;
+        since[c] = i;
+      }
+    }
+    last[c] = i;
+    if (d.kind == kOpRope) {
+      if (rope[c] >= 0 && same_positions(L->ops[rope[c]], d)) d.same_table |= 2;
+      rope[c] = i;
+    }
+  }
+  L->safe = (int32_t)safe;
+}
+
 }  // namespace
 }  // namespace hgk
 
@@ -506,14 +773,10 @@ extern "C" int hgk_op_list_upload(int dtype, const hgk_op* ops, int n_ops, void*
     if (d.kind != kOpRope) continue;
     // the previous rope op's table is still in LDS when this op runs: reuse it
     // when the positions and frequencies are the same
-    if (last_rope >= 0) {
-      const DevOp& p = L->ops[last_rope];
-      d.same_table = p.offsets == d.offsets && p.offset == d.offset && p.scale == d.scale &&
-                     p.half == d.half &&
-                     std::equal(d.inv_freq, d.inv_freq + d.half, p.inv_freq);
-    }
+    if (last_rope >= 0) d.same_table = same_positions(L->ops[last_rope], d);
     last_rope = i;
   }
+  make_chains(L);
   hipError_t e = hipMemcpyAsync(dev_list, host.data(), (size_t)need, hipMemcpyHostToDevice,
                                 as_stream(stream));
   if (e == hipSuccess) e = hipStreamSynchronize(as_stream(stream));
@@ -534,8 +797,12 @@ extern "C" int hgk_op_list_run(int dtype, const void* dev_list, int n_ops, int64
     return fail(HGK_ERR_ARG, "%s: tokens=%lld", fn, (long long)tokens);
   if (tokens == 0) return HGK_OK;
   const DevOpList* L = static_cast<const DevOpList*>(dev_list);
-  const dim3 g((unsigned)tokens), b(kOpThreads);
-  if (dtype == DT_BF16) HGK_LAUNCH((opseq_kernel<BF16>), g, b, 0, as_stream(stream), L, n_ops);
-  else HGK_LAUNCH((opseq_kernel<F16>), g, b, 0, as_stream(stream), L, n_ops);
+  const dim3 b(kOpThreads);
+  // a workgroup per token and chain; where that grid would not fit, one per token
+  const int chained = tokens < ((int64_t)1 << 18);
+  const dim3 g((unsigned)(tokens * (chained ? kChains : 1)));
+  const int nt = (int)tokens;
+  if (dtype == DT_BF16) HGK_LAUNCH((opseq_kernel<BF16>), g, b, 0, as_stream(stream), L, n_ops, nt, chained);
+  else HGK_LAUNCH((opseq_kernel<F16>), g, b, 0, as_stream(stream), L, n_ops, nt, chained);
   return launch_status(fn);
 }

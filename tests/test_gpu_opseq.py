@@ -172,3 +172,85 @@ def test_op_sequence_fewer_tokens_and_a_foreign_list(dev):
     torch.cuda.synchronize()
     for k, v in got[0].items():
         _same_bits(v, before[k], f"foreign list {k}")
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_dependent_ops_over_shared_buffers(dev, seed):
+    """Random lists over a small pool of buffers, so that ops read, overwrite
+    and re-read each other's results (in place, through column slices and
+    through views with another token stride), against the separate calls bit
+    for bit. Chains of dependent ops run in order whatever else runs beside."""
+    T, n, dt = 5, 256, torch.bfloat16
+    r = np.random.default_rng(100 + seed)
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    w = torch.randn(n, generator=g, device=dev).to(dt)
+    base = [torch.randn(T, 2 * n, generator=g, device=dev).to(dt) for _ in range(5)]
+    start = [b.clone() for b in base]
+
+    def view(pool, i, half):  # [T, n]: one half of buffer i's rows
+        return pool[i][:, half * n:(half + 1) * n]
+
+    ops, carry = [], None
+    for _ in range(40):
+        kind = r.choice(["add", "add", "add", "rms", "glu"])
+        a, b, c, d = [(int(r.integers(5)), int(r.integers(2))) for _ in range(4)]
+        if kind == "add" and carry is not None and r.random() < 0.7:
+            a = carry  # the residual stream, sometimes updated in place
+            d = a if r.random() < 0.3 else d
+        if c == d or (kind == "add" and c in (a, b)):
+            continue
+        if kind == "add" and d == b:
+            continue
+        ops.append((kind, a, b, c, d))
+        carry = d if kind == "add" else carry
+    seq = H.OpSequence(dt, torch.device(dev))
+    for kind, a, b, c, d in ops:
+        x, y, out, h = (view(base, *p) for p in (a, b, c, d))
+        if kind == "add":
+            seq.add_rms_norm(x, y, w, 1e-6, out, h)
+        elif kind == "rms":
+            seq.rms_norm(x, w, 1e-6, out)
+        else:
+            seq.glu(ACT_SILU, x, y, out)
+    ref = [b.clone() for b in start]
+    for kind, a, b, c, d in ops:
+        x, y, out, h = (view(ref, *p) for p in (a, b, c, d))
+        if kind == "add":
+            hh, yy = H.add_rms_norm(x.contiguous(), y.contiguous(), w, 1e-6)
+            h.copy_(hh)
+            out.copy_(yy)
+        elif kind == "rms":
+            out.copy_(H.rms_norm(x.contiguous(), w, 1e-6))
+        else:
+            out.copy_(H.swiglu(x.contiguous(), y.contiguous()))
+    for _ in range(2):  # the same list again, from the same start
+        for b, s in zip(base, start):
+            b.copy_(s)
+        seq.run(T)
+        for i, (got, want) in enumerate(zip(base, ref)):
+            assert np.array_equal(to_host(got), to_host(want)), f"buffer {i}"
+
+
+def test_buffers_that_meet_at_a_later_token(dev):
+    """Two ops whose outputs share bytes only from some token on (views with
+    different token strides): up to there they run side by side, over more
+    tokens the list runs in order. Token t of the first op is rows[2 t], of the
+    second rows[8 + t], so token 8's first output is token 8's second."""
+    n, dt = 64, torch.bfloat16
+    g = torch.Generator(device=dev)
+    g.manual_seed(7)
+    x, z = (torch.randn(16, n, generator=g, device=dev).to(dt) for _ in range(2))
+    for T in (8, 12):
+        rows = torch.zeros(40, n, dtype=dt, device=dev)
+        seq = H.OpSequence(dt, torch.device(dev))
+        seq.glu(ACT_SILU, x, z, rows[0:32:2])
+        seq.glu(ACT_SILU, z, x, rows[8:24])
+        seq.run(T)
+        got, a, b = to_host(rows), to_host(H.swiglu(x, z)), to_host(H.swiglu(z, x))
+        # rows one op writes alone, and the row both write for the same token
+        for t in range(T):
+            if not (2 * t - 8 in range(T)):
+                assert np.array_equal(got[2 * t], a[t])
+            if (8 + t) % 2 or (8 + t) // 2 >= T or (8 + t) // 2 == t:
+                assert np.array_equal(got[8 + t], b[t])
