@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
   __shared__ float sxs[8][BM];              // row sums, ring of 8 groups
   // scales and biases of 8 groups per column (double-buffered per 8 groups)
   __shared__ __align__(16) u32x4 ssb[2][kXpBN], bsb[2][kXpBN];
-  __shared__ int32_t list[kGaCap + 4];
+  __shared__ int32_t list[kGaCap + (GEN ? 4 : 0)];
   __shared__ int32_t cnt;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
 
   // this block's part of the pairs
   int64_t scan = 0;
-  const __amdgpu_buffer_rsrc_t rid = buf_rsrc(a.experts, (uint32_t)(a.pairs / 4 * 16));
+  const int64_t all = a.pairs;
   if constexpr (GEN) {
     scan = (int64_t)blockIdx.z * part;
     a.pairs = scan + part < a.pairs ? scan + part : a.pairs;
@@ -1087,6 +1087,8 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
   }
 
   static_assert(RND % 4 == 0, "whole 16-byte id loads");
+  const __amdgpu_buffer_rsrc_t rid = buf_rsrc(a.experts, (uint32_t)(GEN ? all / 4 * 16 : a.pairs * 4));
+
   const uint32_t xbytes = (uint32_t)(((a.xrows - 1) * a.xs + a.K) * 2);
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(a.x, xbytes);
   // the up waves (SW, waves 4-7: also the threads staging the up columns'
