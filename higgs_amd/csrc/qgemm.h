@@ -77,5 +77,8 @@ bool qgemm_few_rows_fits(const QgemmArgs& a);
 // biases 4-byte aligned, a block's rows and columns within 2 GiB.
 bool qgemm_tile_fits(const QgemmArgs& a);
 void qgemm_tile_launch(const QgemmArgs& a, hipStream_t s);
+// 33 to 64 rows, few columns, K a multiple of 2048.
+bool qgemm_tile_split_fits(const QgemmArgs& a);
+void qgemm_tile_split_launch(const QgemmArgs& a, hipStream_t s);
 
 }  // namespace hgk

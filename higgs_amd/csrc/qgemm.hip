@@ -1549,7 +1549,9 @@ bool qgemm_few_rows_fits(const QgemmArgs& a) {
 
 void qgemm_launch(const QgemmArgs& a, hipStream_t s) {
   const unsigned gx = (unsigned)((a.N + kQgBN - 1) / kQgBN);
-  if (a.M <= 64 && decode_fits(a)) {
+  if (qgemm_tile_split_fits(a)) {
+    qgemm_tile_split_launch(a, s);
+  } else if (a.M <= 64 && decode_fits(a)) {
     decode_launch(a, s);
   } else if (qgemm_tile_fits(a)) {
     qgemm_tile_launch(a, s);

@@ -111,7 +111,7 @@ struct TileCfg {
   static constexpr int PART = kTgRing * (XB + CB) + 2 * SB + 2 * 4 * BM * 4;
   static constexpr int LDS = WK * PART;
   static_assert(!PRE || MT % 2 == 0, "the next stage's first row tile goes where row tile 0's was");
-  static_assert(BM * 8 % TP == 0 && BN * 4 % TP == 0 && BN % 64 == 0, "even split of a stage");
+  static_assert(BM * 8 % TP == 0 && BN * 4 % TP == 0 && BN % 32 == 0, "even split of a stage");
   static_assert(BN * 2 % TP == 0 || TP % (BN * 2) == 0, "even split of the codes");
   static_assert(MT % WN == 0 || WN % MT == 0, "row sums split over the column waves");
   // the k-parts' sums, and the output tiles of the waves, meet in the same memory
@@ -424,6 +424,20 @@ bool qgemm_tile_fits(const QgemmArgs& a) {
          256 * a.xs * 2 + a.K * 2 < lim && 256 * a.K / 2 < lim &&
          ((a.M + 63) / 64) * ((a.N + 63) / 64) < lim / 256;
 }
+
+// 33 to 64 rows over few columns: 32 x 32 tiles whose 8 waves split K, where
+// they all run at once. The decode kernel gives a block 16 columns of all rows
+// there, and a CU's x traffic and the chain over K set its time. us, decode
+// kernel / these tiles (N x K): 64 rows 4096 x 12288 55.0 / 27.7, 2048 x 8192
+// 36.5 / 17.3, 4096 x 4096 20.2 / 11.4, 2048 x 2048 10.8 / 7.2; 33 rows 37.9 /
+// 26.3, 24.6 / 16.4, 14.3 / 11.0, 7.7 / 7.1. Up to 32 rows the decode kernel is
+// as fast or faster (17 rows, 2048 x 2048: 6.0 / 7.0), and so it is with more
+// columns (64 rows, 12288 x 4096: 22.6 / 31.8).
+bool qgemm_tile_split_fits(const QgemmArgs& a) {
+  return a.M > 32 && a.M <= 64 && a.K % 2048 == 0 && 2 * ((a.N + 31) / 32) <= 256 && qgemm_tile_fits(a);
+}
+
+void qgemm_tile_split_launch(const QgemmArgs& a, hipStream_t s) { tile_launch<8, 1, 1, 1, 1, false>(a, s); }
 
 // The tile is chosen by the time the launch would take: rounds of resident
 // blocks x groups x the measured time of one group (ns) with 1, 2 or 3 blocks

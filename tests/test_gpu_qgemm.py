@@ -108,6 +108,17 @@ def test_few_rows_take_the_gemv_path(dev, M):
     _check(got, ref, O.BF16, f"M={M}")
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 4096, 2048), (64, 100, 12288), (50, 33, 4096),
+                                   (64, 4097, 2048)], ids=["33-rows", "long-K", "ragged", "wider"])
+def test_decode_rows_over_few_columns(dev, M, N, K):
+    """33 to 64 rows over at most 4096 columns (32 x 32 tiles, K split over 8
+    waves), and one column more (the decode kernel again)."""
+    x, w, s, b = _case(4001 + M + N, M, N, K)
+    got = _run(dev, x, w, s, b, O.BF16)
+    ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
+    _check(got, ref, O.BF16, f"M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 17, 512), (1, 4096, 3584), (2, 1000, 2048), (1, 512, 12288),
                                    (15, 64, 8192), (7, 12289, 512)])
 def test_few_rows_on_the_decode_kernel(dev, M, N, K):
