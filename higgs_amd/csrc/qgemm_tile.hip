@@ -201,11 +201,11 @@ __global__ __launch_bounds__(64 * WK * WM * WN, 2) void qgemm_tile_kernel(QgemmA
   for (int f = 0; f < 4; ++f) ao[f] = arow * 128 + ((4 * lh + f) ^ tg_swizzle(l32)) * 16;
   const int bo = (wn * 32 * NT + l32) * 32 + ((lh ^ (l32 >> 3)) & 1) * 16;
   const int sco = (wn * 32 * NT + l32) * 4;
-  // the row sums' A operand of a 16 x 16 x 32 MFMA: an x fragment (row l32, half lh) read as
-  // its B operand has row c in k-groups 0, 2 and row 16 + c in 1, 3 of column c, so ones in
-  // the even k-groups of the even rows and in the odd ones of the odd rows tell the two apart
-  const uint32_t one = ((lane ^ (lane >> 4)) & 1) ? 0u : 0x3f803f80u;
-  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4{one, one, one, one});
+  // the row sums' B operand of a 16 x 16 x 32 MFMA against ones: rows 0 .. 15 (16 .. 31) of a
+  // row tile in its columns, pieces lg and lg + 4 of them in k-group lg = lane / 16. A column
+  // holds one row of x only, so that an Inf or NaN stays in its own row's sum.
+  const int ro = (wm * 32 * MT + (lane & 15)) * 128 + ((lane >> 4) ^ tg_swizzle(lane & 15)) * 16;
+  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
 
   u32x4 wr[NT];
   bf16x8_t av[2][4];
@@ -278,13 +278,15 @@ __global__ __launch_bounds__(64 * WK * WM * WN, 2) void qgemm_tile_kernel(QgemmA
 #pragma unroll
         for (int q = 0; q < C::Q; ++q) {
           const int rt = (wn * C::Q + q) % MT;
-          f32x4_t sx = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+          f32x4_t sx[2] = {};
 #pragma unroll
-          for (int f = 0; f < 4; ++f)
-            sx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                ones, *reinterpret_cast<const bf16x8_t*>(xb + ao[f] + rt * 4096), sx, 0, 0, 0);
-          // lanes 0 .. 31: the sum of row l32
-          if (lh == 0) sums[(sbuf * 4 + j) * C::BM + wm * 32 * MT + rt * 32 + l32] = (lane & 16) ? sx[1] : sx[0];
+          for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              sx[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  ones, *reinterpret_cast<const bf16x8_t*>(xb + (ro ^ (64 * f)) + h * 2048 + rt * 4096), sx[h], 0, 0, 0);
+          // every row of a result is the same: lanes 0 .. 31 take the sum of row l32
+          if (lh == 0) sums[(sbuf * 4 + j) * C::BM + wm * 32 * MT + rt * 32 + l32] = (lane & 16) ? sx[1][0] : sx[0][0];
         }
       }
       __builtin_amdgcn_sched_barrier(0);

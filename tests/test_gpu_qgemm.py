@@ -88,6 +88,27 @@ def test_tile_sizes(dev, M, N, K, ys):
     _check(got[:, :N][np.ix_(rows, cols)], ref, O.BF16, f"M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 512, 2048), (64, 4096, 2048), (40, 8200, 2048),
+                                   (129, 200, 1024), (301, 1001, 512), (1024, 2048, 512),
+                                   (700, 12288, 512), (4100, 12288, 512)],
+                         ids=["33-rows", "split-K", "decode", "64x64", "64x128x2", "64x128",
+                              "128x128", "256x256"])
+def test_a_row_with_inf_or_nan_leaves_the_others(dev, M, N, K):
+    """Rows of x do not meet: with an Inf or NaN in the first and last rows, in
+    a row and in the row 16 after it, every other row keeps its bits."""
+    x, w, s, b = _case(3851 + M + N, M, N, K)
+    clean = _run(dev, x, w, s, b, O.BF16)
+    bad = [0, 3, 20, M - 1]
+    x = x.copy()
+    for r, v in zip(bad, (0x7F80, 0x7FC0, 0xFF80, 0x7F80)):  # Inf, NaN, -Inf, Inf
+        x[r, (37 * r + 5) % K] = v
+    got = _run(dev, x, w, s, b, O.BF16)
+    rest = np.setdiff1d(np.arange(M), bad)
+    assert np.array_equal(got[rest], clean[rest])
+    # an Inf meets weights of both signs and a few zeros: no output is finite
+    assert ((got[bad] & 0x7F80) == 0x7F80).mean() > 0.99
+
+
 def test_qwen3_next_prefill_projection(dev):
     """A 2048-token prefill through a 2048 -> 4096 projection (the attention
     q projection's shape class)."""
