@@ -64,11 +64,11 @@ __device__ inline uint32_t lds_addr(const void* p) {
 // dst and soff are wave-uniform.
 __device__ inline void dma16(uint32_t dst, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(dst), "v"(voff), "s"(r), "s"(soff) : "memory");
+               :: "s"(dst), "v"(voff), "s"(r), "s"(soff) : "m0", "memory");
 }
 __device__ inline void dma4(uint32_t dst, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :: "s"(dst), "v"(voff), "s"(r), "s"(soff) : "memory");
+               :: "s"(dst), "v"(voff), "s"(r), "s"(soff) : "m0", "memory");
 }
 
 // all but the newest N loads of this wave have landed, then the block's barrier
