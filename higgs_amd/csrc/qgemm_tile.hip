@@ -61,7 +61,11 @@ __device__ inline uint32_t lds_addr(const void* p) {
 }
 
 // 16 (or 4) bytes per lane from rsrc + voff + soff to LDS at dst + 16 (4) * lane.
-// dst and soff are wave-uniform.
+// dst and soff are wave-uniform. m0 is a register that the compiler reserves: it never holds a
+// value of its own there for long, but may move or merge its writes to it, so it has to know of
+// this one (and need not warn that nothing preserves it).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ inline void dma16(uint32_t dst, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :: "s"(dst), "v"(voff), "s"(r), "s"(soff) : "m0", "memory");
@@ -70,6 +74,8 @@ __device__ inline void dma4(uint32_t dst, __amdgpu_buffer_rsrc_t r, uint32_t vof
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                :: "s"(dst), "v"(voff), "s"(r), "s"(soff) : "m0", "memory");
 }
+
+#pragma clang diagnostic pop
 
 // all but the newest N loads of this wave have landed, then the block's barrier
 template <int N>

@@ -109,6 +109,35 @@ def test_a_row_with_inf_or_nan_leaves_the_others(dev, M, N, K):
     assert ((got[bad] & 0x7F80) == 0x7F80).mean() > 0.99
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 300, 2048), (129, 200, 1024), (301, 1001, 512),
+                                   (1024, 2048, 512), (700, 12288, 512), (4100, 12288, 512)],
+                         ids=["split-K", "64x64", "64x128x2", "64x128", "128x128", "256x256"])
+def test_tiles_keep_the_sign_of_an_inf(dev, M, N, K):
+    """What the tiles' group form cannot hold comes out as the f32 sum has it: a
+    row with one Inf gives Inf with the sign of its weight, a row with one value
+    whose product with a code overflows gives that value's finite result, an Inf
+    bias gives Inf with the sign of its group's sum of x. The rest keeps its
+    bits."""
+    x, w, s, b = _case(3871 + M + N, M, N, K)
+    clean = _run(dev, x, w, s, b, O.BF16)
+    x, b = x.copy(), b.copy()
+    inf, big, k, col, g = 2, M - 1, 70, min(77, N - 1), 3
+    x[inf, k] = 0x7F80
+    x[big, k] = 0x7F60  # 2.98e38
+    b[col, g] = 0xFF80
+    got = _run(dev, x, w, s, b, O.BF16)
+    rows, cols = np.setdiff1d(np.arange(M), [inf, big]), np.setdiff1d(np.arange(N), [col])
+    assert np.array_equal(got[np.ix_(rows, cols)], clean[np.ix_(rows, cols)])
+    q = (w[:, k // 8] >> np.uint32(4 * (k % 8))) & 15
+    wk = (O.to_f32(s[:, k // 64], O.BF16) * q.astype(np.float32) + O.to_f32(b[:, k // 64], O.BF16))[cols]
+    want = np.where(wk == 0, np.nan, np.copysign(np.inf, wk))
+    assert np.array_equal(O.to_f32(got[inf, cols], O.BF16), want, equal_nan=True)
+    large = O.from_f32((O.to_f32(x[big, k], O.BF16) * wk).astype(np.float32), O.BF16)
+    _check(got[big, cols][wk != 0], large[wk != 0], O.BF16, "one large value")
+    sx = O.to_f32(x[rows, 64 * g:64 * g + 64], O.BF16).sum(1)
+    assert np.array_equal(O.to_f32(got[rows, col], O.BF16), np.copysign(np.inf, -sx))
+
+
 def test_qwen3_next_prefill_projection(dev):
     """A 2048-token prefill through a 2048 -> 4096 projection (the attention
     q projection's shape class)."""
