@@ -104,6 +104,64 @@ __device__ inline bf16x8_t tg_expand(uint32_t c) {
 // that neither 8 nor 16 consecutive lanes of a fragment read share a bank.
 __device__ inline int tg_swizzle(int r) { return ((r >> 1) & 3) | (((r ^ (r >> 3)) & 1) << 2); }
 
+// The Inf and NaN outputs of a wave's tile (rows m0 .., columns n0 ..; at most 64 columns), again
+// in plain f32. The group form meets an Inf of x with the zero codes and with b Sx of the other
+// sign, an Inf bias with the zero parts of Sx, and products x q may overflow where x w does not:
+// NaN where the sum is Inf or finite. So an output of finite scales and biases is sum x (s q + b)
+// in f32, as the GEMV has it, and one with others the sum of s C + b Sx per group. Rows that hold a
+// NaN are NaN in every column already. The outputs are read past the L1, which a neighbour's read
+// of the same line may have filled before this wave's stores.
+__device__ inline void tg_redo(const QgemmArgs& a, int64_t m0, int rows, int64_t n0, int cols, int lane) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int64_t KW = a.K / 8, G = a.K / 64;
+  for (int64_t m = m0; m < m0 + rows && m < a.M; ++m) {
+    uint32_t v = 0;
+    if (lane < cols && n0 + lane < a.N)
+      v = __hip_atomic_load(a.y + m * a.ys + n0 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint64_t todo = __ballot((v & 0x7f80u) == 0x7f80u);
+    if (!todo) continue;
+    const uint16_t* xr = a.x + m * a.xs;
+    bool nan = false;
+    for (int64_t k = 8 * lane; k < a.K; k += 512) {
+      const u32x4 q = *reinterpret_cast<const u32x4*>(xr + k);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) nan |= (q[i] & 0x7fffu) > 0x7f80u || (q[i] & 0x7fff0000u) > 0x7f800000u;
+    }
+    if (__ballot(nan)) continue;
+    for (; todo; todo &= todo - 1) {
+      const int64_t n = n0 + __builtin_ctzll(todo);
+      float each = 0.0f, grouped = 0.0f;
+      bool finite = true;
+      for (int64_t c = lane; c < KW; c += 64) {  // K a multiple of 512: the same count in every lane
+        const uint32_t q = a.w[n * KW + c];
+        const u32x4 xq = *reinterpret_cast<const u32x4*>(xr + 8 * c);
+        const uint32_t su = a.sc[n * G + c / 8], bu = a.bi[n * G + c / 8];
+        const float s = BF16::lo(su), b = BF16::lo(bu);
+        finite &= (su & 0x7f80u) != 0x7f80u && (bu & 0x7f80u) != 0x7f80u;
+        float cq = 0.0f, sx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float x = i & 1 ? BF16::hi(xq[i / 2]) : BF16::lo(xq[i / 2]), qf = (float)((q >> (4 * i)) & 15u);
+          each = __builtin_fmaf(x, __builtin_fmaf(s, qf, b), each);
+          cq = __builtin_fmaf(x, qf, cq);
+          sx += x;
+        }
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) {
+          cq += __shfl_xor(cq, o, 64);
+          sx += __shfl_xor(sx, o, 64);
+        }
+        grouped = __builtin_fmaf(s, cq, __builtin_fmaf(b, sx, grouped));
+      }
+      each = group_sum<64>(each);
+#pragma unroll
+      for (int o = 8; o < 64; o <<= 1) grouped += __shfl_xor(grouped, o, 64);
+      const float r = __ballot(!finite) ? grouped : each;
+      if (lane == 0) a.y[m * a.ys + n] = (uint16_t)(BF16::pack(r, 0.0f) & 0xffffu);
+    }
+  }
+}
+
 template <int WK, int WM, int WN, int MT, int NT, bool PRE>
 struct TileCfg {
   static constexpr int TP = 64 * WM * WN;       // threads of a k-part
@@ -386,6 +444,7 @@ __global__ __launch_bounds__(64 * WK * WM * WN, 2) void qgemm_tile_kernel(QgemmA
   constexpr int PITCH = NT * 64 + 16, PCS = NT * 4;  // bytes and 16-byte pieces per row
   unsigned char* const ob = lds + wv * 32 * PITCH;
   const bool vec = (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && a.ys % 8 == 0;
+  uint32_t bad = 0;  // bit 15 or 31: an Inf or NaN
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
 #pragma unroll
@@ -401,6 +460,8 @@ __global__ __launch_bounds__(64 * WK * WM * WN, 2) void qgemm_tile_kernel(QgemmA
       const u32x4 v = *reinterpret_cast<const u32x4*>(ob + row * PITCH + cp * 16);
       const int64_t m = m0 + wm * 32 * MT + i * 32 + row, n = n0 + wn * 32 * NT + cp * 8;
       if (m < a.M) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) bad |= (v[k] & 0x7f807f80u) + 0x00800080u;
         uint16_t* const yp = a.y + m * a.ys + n;
         if (vec && n + 8 <= a.N) {
           *reinterpret_cast<u32x4*>(yp) = v;
@@ -413,6 +474,7 @@ __global__ __launch_bounds__(64 * WK * WM * WN, 2) void qgemm_tile_kernel(QgemmA
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
+  if (__ballot(bad & 0x80008000u)) tg_redo(a, m0 + wm * 32 * MT, 32 * MT, n0 + wn * 32 * NT, 32 * NT, lane);
 }
 
 template <int WK, int WM, int WN, int MT, int NT, bool PRE>
