@@ -53,17 +53,21 @@ void gather_grouped_launch(const GatherArgs& a, hipStream_t s);
 // bi2: up, same shapes); false where the fused kernel does not apply.
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s);
 
-// Rows of x at or above which the MFMA kernels run for every K. Below, they
-// run where the decode kernel takes the call (K a multiple of 512, scales and
-// biases 4-byte aligned): it reads each weight once for all rows, while the
-// GEMV kernels read them once per row (and, for K other than 512, 1024, 2048
-// and 4096, one element at a time: 80 us at 1 x 4096 x 12288 against 20).
+// Rows of x at or above which the MFMA kernels run for every K. Below:
+// - 2 to 15 rows where the one-row GEMV has K (512, 1024, 2048 or 4096): the
+//   decode kernel's form for few rows, which reads each weight once for all of
+//   them; its f32 sums are no less exact than the GEMV's (see there);
+// - one row: the GEMV;
+// - other K: qmv_chain_kernel or the generic kernel (qmm.hip), whose sums of
+//   x (s q + b) no group form reaches where x has a mean.
 // us per call, GEMV / decode kernel:
 //   N x K           1 row         4 rows        15 rows
-//   12288 x 4096    12.8 / 11.8   23.6 / 12.3   59.7 / 13.7
-//   12288 x 2048    7.5 / 6.9     11.2 / 6.9    25.9 / 7.3
-//   2048 x 2048     5.4 / 4.6     5.5 / 4.9     7.5 / 5.5
-//   512 x 2048      4.7 / 4.3     4.8 / 4.6     5.0 / 5.2
+//   12288 x 4096    12.6 / 11.6   23.5 / 12.2   60.5 / 13.5
+//   12288 x 2048    6.3 / 6.5     10.1 / 6.7    25.4 / 7.2
+//   4096 x 4096     9.7 / 7.9     10.1 / 8.1    23.9 / 9.6
+//   2048 x 2048     5.4 / 5.9     5.4 / 6.0     7.4 / 5.8
+// (One row is 8 to 20 % slower with K 4096 than on the decode kernel, and
+// gives the bits that gather_qmm gives for the same row.)
 constexpr int64_t kQgemmMinRows = 16;
 
 // bf16 activations and scales, group 64, 4 bits, x 16-byte aligned with a

@@ -61,6 +61,22 @@ __device__ inline bf16x8_t expand_codes(uint32_t c) {
   return __builtin_bit_cast(bf16x8_t, v);
 }
 
+// 8 codes of one word -> the bf16 numbers q in order. A byte 0 .. 15 read as
+// fp8 (e4m3) is q * 2^-9 exactly (subnormals up to 7, the first binade from
+// 8), so the scaled conversion gives q itself.
+__device__ inline bf16x8_t expand_q(uint32_t c) {
+  const uint32_t lo = c & 0x0f0f0f0fu;         // q0 q2 q4 q6
+  const uint32_t hi = (c >> 4) & 0x0f0f0f0fu;  // q1 q3 q5 q7
+  const uint32_t p = __builtin_amdgcn_perm(hi, lo, 0x05010400u);  // q0 q1 q2 q3
+  const uint32_t q = __builtin_amdgcn_perm(hi, lo, 0x07030602u);  // q4 q5 q6 q7
+  u32x4 v;
+  v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(p, 512.0f, false));
+  v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(p, 512.0f, true));
+  v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q, 512.0f, false));
+  v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q, 512.0f, true));
+  return __builtin_bit_cast(bf16x8_t, v);
+}
+
 // 8 codes of one word -> the bf16 numbers 128 + q in the order (q0, q4),
 // (q1, q5), (q2, q6), (q3, q7): for x stored in the same order, each pair is
 // one shift and one and-or (7 operations per word against 11 above).
@@ -285,7 +301,16 @@ __device__ inline __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, uint32_t bytes)
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, kBufWord3);
 }
 
-template <int MT, int NT, int MS>
+//
+// FEW (2 to 15 rows): the codes as q (expand_q), and the affine part in f32 per
+// group, acc += s (x . q) and acc += b Sx, with the row sums from x against
+// ones (lane (l16, lg) gets those of its rows 4 lg + r). With 128 + q a sum
+// holds x (128 + q) until 128 Sx is taken off, and its f32 rounding shows: rms
+// error of outputs next to zero over the rms of all outputs, 15 x 65536 x 2048,
+// x of unit deviation and mean 0 / 1 / 4: 1.6e-6 / - / 1.3e-5 with 128 + q,
+// 0.8e-7 / 1.8e-7 / 1.8e-7 in this form, 4.8e-7 / 1.6e-6 / 1.8e-7 in the
+// one-row GEMV.
+template <int MT, int NT, int MS, bool FEW>
 __global__ __launch_bounds__(kDecThreads) void qgemm_decode_kernel(QgemmArgs a) {
   constexpr int ROWS = 16 * NT;
   constexpr int WB = ROWS * kDecPitch;             // codes of a chunk
@@ -405,31 +430,36 @@ __global__ __launch_bounds__(kDecThreads) void qgemm_decode_kernel(QgemmArgs a) 
     auto compute = [&](const DecX<MT>& q, int s) {
       const int gl = 8 * s + wave;  // group within the chunk
       bf16x8_t bw[NT][2];
-      float sc[NT];
+      float sc[NT], bi[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int row = t * 16 + l16;
         const unsigned char* wp = lds + row * kDecPitch + gl * 32 + lg * 4;
         uint32_t w0 = *reinterpret_cast<const uint32_t*>(wp), w1 = *reinterpret_cast<const uint32_t*>(wp + 16);
         asm volatile("" : "+v"(w0), "+v"(w1));
-        bw[t][0] = expand_codes(w0);
-        bw[t][1] = expand_codes(w1);
+        bw[t][0] = FEW ? expand_q(w0) : expand_codes(w0);
+        bw[t][1] = FEW ? expand_q(w1) : expand_codes(w1);
         sc[t] = BF16::lo(*reinterpret_cast<const uint16_t*>(sct + row * (kDecCG * 2) + gl * 2));
+        if constexpr (FEW) bi[t] = BF16::lo(*reinterpret_cast<const uint16_t*>(bit + row * (kDecCG * 2) + gl * 2));
       }
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
         const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, q.x[i][0]);
         const bf16x8_t a1 = __builtin_bit_cast(bf16x8_t, q.x[i][1]);
-        // ones . x^T: every output of lane (l16, lg) is the row sum of row l16
-        f32x4_t sx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, a0, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-        sx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, a1, sx, 0, 0, 0);
+        // ones . x^T: every output of lane (l16, lg) is the row sum of row l16 (FEW: x . ones^T)
+        f32x4_t sx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(FEW ? a0 : ones, FEW ? ones : a0,
+                                                             f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        sx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(FEW ? a1 : ones, FEW ? ones : a1, sx, 0, 0, 0);
         sxs[s][i] = sx[0];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           f32x4_t c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bw[t][0], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
           c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, bw[t][1], c, 0, 0, 0);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][t][r] = __builtin_fmaf(sc[t], c[r], acc[i][t][r]);
+          for (int r = 0; r < 4; ++r) {
+            acc[i][t][r] = __builtin_fmaf(sc[t], c[r], acc[i][t][r]);
+            if constexpr (FEW) acc[i][t][r] = __builtin_fmaf(bi[t], sx[r], acc[i][t][r]);
+          }
         }
         // the tile row's update completes here (otherwise every MFMA result
         // of the group is held at once)
@@ -460,6 +490,7 @@ __global__ __launch_bounds__(kDecThreads) void qgemm_decode_kernel(QgemmArgs a) 
         fetch_x(xr[s & 1], s + 2);
       }
     }
+    if constexpr (FEW) continue;
     // bias term of the wave's 4 groups, sum_g (b - 128 s)[n, g] Sx_g[m], as one
     // f32 MFMA (16 x 16 x 4) per tile: k = the sub-chunk, lane (l16, lg)
     // supplies Sx of row l16 and (b - 128 s) of column l16 for sub-chunk lg
@@ -1484,13 +1515,13 @@ void gather_grouped_launch(const GatherArgs& a, hipStream_t s) {
 }
 
 
-template <int MT>
+template <int MT, bool FEW = false>
 void decode_launch_mt(const QgemmArgs& a, int nt, hipStream_t s) {
   const dim3 grid((unsigned)((a.N + 16 * nt - 1) / (16 * nt))), block(kDecThreads);
   switch (nt) {
-    case 1: HGK_LAUNCH((qgemm_decode_kernel<MT, 1, 1>), grid, block, 0, s, a); break;
-    case 2: HGK_LAUNCH((qgemm_decode_kernel<MT, 2, 1>), grid, block, 0, s, a); break;
-    default: HGK_LAUNCH((qgemm_decode_kernel<MT, 3, 1>), grid, block, 0, s, a); break;
+    case 1: HGK_LAUNCH((qgemm_decode_kernel<MT, 1, 1, FEW>), grid, block, 0, s, a); break;
+    case 2: HGK_LAUNCH((qgemm_decode_kernel<MT, 2, 1, FEW>), grid, block, 0, s, a); break;
+    default: HGK_LAUNCH((qgemm_decode_kernel<MT, 3, 1, FEW>), grid, block, 0, s, a); break;
   }
 }
 
@@ -1522,12 +1553,13 @@ void decode_launch(const QgemmArgs& a, hipStream_t s) {
     const int64_t tiles = (a.N + 16 * NT - 1) / (16 * NT);
     if (2 * tiles >= kCUs) {
       const dim3 grid((unsigned)(((tiles + 7) / 8) * 16)), block(kDecThreads);
-      HGK_LAUNCH((qgemm_decode_kernel<2, NT, 2>), grid, block, 0, s, a);
+      HGK_LAUNCH((qgemm_decode_kernel<2, NT, 2, false>), grid, block, 0, s, a);
       return;
     }
   }
   int nt = 3;
   while (nt > 1 && (a.N + 16 * nt - 1) / (16 * nt) < kCUs) --nt;
+  if (a.M < kQgemmMinRows) return decode_launch_mt<1, true>(a, nt, s);
   switch ((a.M + 15) / 16) {
     case 1: decode_launch_mt<1>(a, nt, s); break;
     case 2: decode_launch_mt<2>(a, nt, s); break;
@@ -1544,7 +1576,9 @@ bool qgemm_supported(int dtype, int sdt, int group_size, int bits, const void* x
 }
 
 bool qgemm_few_rows_fits(const QgemmArgs& a) {
-  return decode_fits(a) && ((reinterpret_cast<uintptr_t>(a.sc) | reinterpret_cast<uintptr_t>(a.bi)) & 3) == 0;
+  return a.M > 1 && (a.K == 512 || a.K == 1024 || a.K == 2048 || a.K == 4096) && decode_fits(a) &&
+         (reinterpret_cast<uintptr_t>(a.w) & 15) == 0 &&
+         ((reinterpret_cast<uintptr_t>(a.sc) | reinterpret_cast<uintptr_t>(a.bi)) & 3) == 0;
 }
 
 void qgemm_launch(const QgemmArgs& a, hipStream_t s) {

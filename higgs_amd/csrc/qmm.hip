@@ -288,7 +288,142 @@ __global__ __launch_bounds__(256) void qmv_generic_kernel(QmmArgs a) {
   }
 }
 
+// quantized_matmul of 1 to 15 rows with group 64 and K a multiple of 512 that
+// the kernels above do not have (3584, 8192, 12288, ...): the generic kernel's
+// arithmetic, operation by operation, from wide loads. There lane l of an
+// output's wave sums x[k] (s q + b) over k = l, l + 64, ..., one product per
+// group, and the 64 sums meet in a tree of lane distances 32, 16, .. 1; here a
+// lane has four of those sums (codes 4 h .. 4 h + 3 of each group, h = lane %
+// 16) of one output of R rows, a wave 4 outputs. s q is exact, so one fma
+// rounds as the product and the sum do: the same bits.
+//
+// A wave walks its columns' codes in stages of 8 groups: 16-byte loads (256
+// contiguous bytes per column), four stages in flight in registers; a stage
+// goes through the wave's own LDS slice, where each lane picks its 2 bytes per
+// group (4 columns x 32 consecutive bytes: no bank twice). The block's x goes
+// to LDS as f32, 32 groups at a time, double-buffered: one barrier per 32
+// groups. One row is bound by 17 vector instructions per 4 codes (5.5 us for
+// 50 M codes); each further row adds 4 and a 16-byte LDS read. us, generic
+// kernel (a row at a time, a 4-byte load per code) / this one:
+//   N x K           1 row         4 rows        15 rows
+//   4096 x 12288    97.8 / 15.3   208 / 22.9    704 / 52.3
+//   3584 x 14336    113 / 16.6    220 / 25.7    725 / 58.7
+//   14336 x 3584    68.1 / 11.9   208 / 21.8    732 / 65.7
+//   2048 x 8192     39.6 / 9.7    72.2 / 15.7   235 / 20.3
+template <int R>
+__global__ __launch_bounds__(256) void qmv_chain_kernel(QmmArgs a) {
+  constexpr int KC = 2048, D = 4;  // elements of x per chunk; stages in flight (a chunk is D stages)
+  static_assert(KC == D * 512, "a chunk's stages");
+  __shared__ __align__(16) float xs[2][R][KC];
+  __shared__ __align__(16) u32x4 cs[4][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int h = lane & 15, c = lane >> 4;
+  const int64_t nw = ((int64_t)blockIdx.x * 4 + wave) * 4;  // the wave's first column
+  const int64_t m0 = (int64_t)blockIdx.y * R;
+  const int S = (int)(a.K / 512);
+  const int64_t G = a.K / 64;
+
+  // lane p loads piece p of a stage: group p / 8, half p % 2 of column p / 2 % 4
+  const int64_t lc = nw + ((lane >> 1) & 3), sc = nw + c;
+  const u32x4* wp = reinterpret_cast<const u32x4*>(a.w + (lc < a.N ? lc : a.N - 1) * (a.K / 8)) +
+                    (lane >> 3) * 2 + (lane & 1);
+  const int64_t srow = (sc < a.N ? sc : a.N - 1) * G;
+  const u32x4* sp = reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.sc) + srow);
+  const u32x4* bp = reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.bi) + srow);
+  u32x4 cq[D], sq[D], bq[D];
+  auto load = [&](int d, int st) {  // past the last stage: the last again
+    const int t = st < S ? st : S - 1;
+    cq[d] = wp[t * 16];
+    sq[d] = sp[t];
+    bq[d] = bp[t];
+  };
+  u32x4 xr[R];
+  auto load_x = [&](int chunk) {
+    const int64_t k = (int64_t)chunk * KC + 8 * tid;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t m = m0 + r < a.pairs ? m0 + r : a.pairs - 1;
+      xr[r] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.x) + m * a.xs +
+                                              (k < a.K ? k : a.K - 8));
+    }
+  };
+  auto publish_x = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float* p = &xs[buf][r][8 * tid];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[2 * i] = BF16::lo(xr[r][i]);
+        p[2 * i + 1] = BF16::hi(xr[r][i]);
+      }
+    }
+  };
+
+  float acc[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[r][i] = 0.0f;
+
+  load_x(0);
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+  publish_x(0);
+  load_x(1);
+  for (int s0 = 0, buf = 0; s0 < S; s0 += D, buf ^= 1) {
+    __syncthreads();  // this chunk's x is there; the other buffer's readers are done
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (s0 + d >= S) break;
+      cs[wave][lane] = cq[d];  // in order behind the reads of the stage before, of this wave alone
+      const u32x4 sv = sq[d], bv = bq[d];
+      load(d, s0 + d + D);
+      const unsigned char* cb = reinterpret_cast<const unsigned char*>(cs[wave]) + c * 32 + h * 2;
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const uint32_t q = *reinterpret_cast<const uint16_t*>(cb + g * 128);
+        const uint32_t lo = q & 0x0f0fu, hi = (q >> 4) & 0x0f0fu;
+        const float s = g & 1 ? BF16::hi(sv[g / 2]) : BF16::lo(sv[g / 2]);
+        const float b = g & 1 ? BF16::hi(bv[g / 2]) : BF16::lo(bv[g / 2]);
+        float w[4];
+        w[0] = __builtin_fmaf(s, (float)(lo & 0xffu), b);
+        w[1] = __builtin_fmaf(s, (float)(hi & 0xffu), b);
+        w[2] = __builtin_fmaf(s, (float)(lo >> 8), b);
+        w[3] = __builtin_fmaf(s, (float)(hi >> 8), b);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const float* xp = &xs[buf][r][(d * 8 + g) * 64 + h * 4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[r][i] = __builtin_fmaf(xp[i], w[i], acc[r][i]);
+        }
+      }
+    }
+    publish_x(buf ^ 1);
+    load_x(s0 / D + 2);
+  }
+
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[r][i] += __shfl_xor(acc[r][i], o, 64);
+    const float v = (acc[r][0] + acc[r][2]) + (acc[r][1] + acc[r][3]);
+    if (h == 0 && sc < a.N && m0 + r < a.pairs) store1<BF16>(a.y, (m0 + r) * a.ys + sc, v);
+  }
+}
+
 namespace {
+
+void launch_chain(const QmmArgs& a, hipStream_t s) {
+  const int r = a.pairs == 1 ? 1 : a.pairs == 2 ? 2 : 4;
+  const dim3 grid((unsigned)((a.N + 15) / 16), (unsigned)((a.pairs + r - 1) / r));
+  switch (r) {
+    case 1: HGK_LAUNCH((qmv_chain_kernel<1>), grid, dim3(256), 0, s, a); break;
+    case 2: HGK_LAUNCH((qmv_chain_kernel<2>), grid, dim3(256), 0, s, a); break;
+    default: HGK_LAUNCH((qmv_chain_kernel<4>), grid, dim3(256), 0, s, a); break;
+  }
+}
 
 template <class S, int STEPS>
 void launch_bf16_k(QmmArgs a, hipStream_t s) {
@@ -443,6 +578,10 @@ extern "C" int hgk_quantized_matmul(int dtype, const void* x, int64_t m, int64_t
   const bool vec_ok = dtype == DT_BF16 && aligned16(x) && x_row_stride % 8 == 0 && aligned16(w) &&
                       (reinterpret_cast<uintptr_t>(scales) & 1) == 0;
   if (vec_ok && launch_bf16<BF16>(a, s)) return launch_status(fn);
+  if (vec_ok && m < kQgemmMinRows && group_size == 64 && k % 512 == 0 && aligned16(scales) && aligned16(biases)) {
+    launch_chain(a, s);
+    return launch_status(fn);
+  }
   if (dtype == DT_BF16) launch_generic<BF16, BF16>(a, s);
   else launch_generic<F16, F16>(a, s);
   return launch_status(fn);

@@ -401,9 +401,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
     """quantized_matmul(x, w, scales, biases, transpose, group_size, bits) as
     QLinear::forward calls it (qwen3_next.rs:174-221): x [..., K], w [N,
     K*bits/32] packed 32-bit words, scales/biases [N, K/group_size]. Returns
-    y [..., N] in x's dtype. bf16 with group 64 runs on the matrix cores (fewer
-    than 16 rows: where K is a multiple of 512); f16, other groups and the rest
-    run one GEMV per row."""
+    y [..., N] in x's dtype. bf16 with group 64 runs on the matrix cores from 16
+    rows on, and from 2 rows where K is 512, 1024, 2048 or 4096; fewer rows, f16
+    and other groups run on the GEMV kernels."""
     if not transpose:
         raise HgkError(2, "quantized_matmul: only transpose=True (weights stored [N, K]) is implemented")
     if w.dim() != 2 or scales.dim() != 2 or scales.shape != biases.shape:

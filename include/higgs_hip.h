@@ -297,8 +297,9 @@ int hgk_gather_qmm_swiglu(int dtype, const void* x, int64_t x_rows, int64_t x_ro
  * stride) in `dtype`; w [N, K*bits/32] u32; scales/biases [N, K/group_size]
  * in scales_dtype; y [M, N] (row stride y_row_stride). bits = 4,
  * group_size 32, 64 or 128, bf16 or f16 with scales of the same dtype. With
- * bf16 and group 64 the matrix cores run it (M >= 16, or K a multiple of 512;
- * exact products, f32 sums, one rounding); otherwise one GEMV per row.
+ * bf16 and group 64 the matrix cores run it (M >= 16, or M >= 2 and K 512,
+ * 1024, 2048 or 4096; exact products, f32 sums, one rounding); otherwise the
+ * GEMV kernels.
  */
 int hgk_quantized_matmul(int dtype, const void* x, int64_t m, int64_t x_row_stride,
                          const uint32_t* w, const void* scales, const void* biases,

@@ -2,9 +2,9 @@
 against the oracle (the exact f64 contraction rounded once). A floating-point
 contraction accumulated in f32, so the bar is the stated tolerance, written
 here: every bf16/f16 output within 1 ulp of the oracle, or within atol 1e-3
-next to zero (rtol 1e-2, atol 1e-3); at least 99 % bit-identical. M >= 16
-rows in bf16 with group 64 run on the matrix cores; the rest one GEMV per
-row."""
+next to zero (rtol 1e-2, atol 1e-3); at least 99 % bit-identical. bf16
+with group 64 runs on the matrix cores from 16 rows on, and from 2 with K 512,
+1024, 2048 or 4096; the rest on the GEMV kernels."""
 from __future__ import annotations
 
 import numpy as np
@@ -151,7 +151,7 @@ def test_qwen3_next_prefill_projection(dev):
 
 
 @pytest.mark.parametrize("M", [1, 3, 15])
-def test_few_rows_take_the_gemv_path(dev, M):
+def test_few_rows(dev, M):
     x, w, s, b = _case(3200 + M, M, 512, 2048)
     got = _run(dev, x, w, s, b, O.BF16)
     ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
@@ -171,13 +171,72 @@ def test_decode_rows_over_few_columns(dev, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 17, 512), (1, 4096, 3584), (2, 1000, 2048), (1, 512, 12288),
                                    (15, 64, 8192), (7, 12289, 512)])
-def test_few_rows_on_the_decode_kernel(dev, M, N, K):
-    """1 to 15 rows with K a multiple of 512: column tiles that are partly
-    filled, K beyond the GEMV's list, few and many column tiles."""
+def test_few_rows_of_any_k(dev, M, N, K):
+    """1 to 15 rows: column tiles that are partly filled, K beyond the GEMV's
+    list, few and many column tiles."""
     x, w, s, b = _case(3901 + M + N, M, N, K)
     got = _run(dev, x, w, s, b, O.BF16)
     ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
     _check(got, ref, O.BF16, f"M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 300, 512), (1, 130, 4096), (1, 35, 1536), (2, 17, 2560),
+                                   (3, 64, 3584), (4, 100, 8192), (5, 33, 1536), (15, 48, 12288),
+                                   (9, 70, 576), (1, 40, 14336)])
+def test_few_rows_have_the_per_pair_kernels_bits(dev, M, N, K):
+    """One row, and 1 to 15 rows with K outside 512, 1024, 2048 and 4096, are the
+    per-pair kernels' sums operation by operation: the bits of gather_qmm over
+    one expert, also for rows with an Inf or NaN."""
+    x, w, s, b = _case(4101 + M + N, M, N, K)
+    for bad in (None, 0x7F80, 0x7FC0):
+        if bad is not None:
+            x = x.copy()
+            x[M - 1, K - 70] = bad
+        y = to_host(H.gather_qmm(to_dev(x, O.BF16, dev), words_dev(w, dev)[None],
+                                 to_dev(s, O.BF16, dev)[None], to_dev(b, O.BF16, dev)[None],
+                                 torch.zeros(M, dtype=torch.int32, device=dev)))
+        got = _run(dev, x, w, s, b, O.BF16)
+        nan = np.isnan(O.to_f32(y, O.BF16))
+        assert np.array_equal(np.isnan(O.to_f32(got, O.BF16)), nan)
+        assert np.array_equal(got[~nan], y[~nan])
+
+
+def sum_error(y, x, w, s, b):
+    """The f32 sums' error: the rms error of the outputs within 1e-4 of the rms of
+    all (their bf16 rounding is below 1e-7 of it), over that rms."""
+    sh = torch.arange(0, 32, 4, device=w.device, dtype=torch.int32)
+    q = ((w.unsqueeze(-1) >> sh) & 15).flatten(-2).double()
+    wd = q * s.double().repeat_interleave(64, -1) + b.double().repeat_interleave(64, -1)
+    ref = x.double() @ wd.t()
+    rms = ref.pow(2).mean().sqrt()
+    near = ref.abs() < 1e-4 * rms
+    assert int(near.sum()) >= 20
+    return float(((y.double() - ref)[near] / rms).pow(2).mean().sqrt())
+
+
+def random_projection(g, dev, N, K):
+    """Codes, scales and biases of weights with a mean near zero."""
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), dtype=torch.int32, device=dev, generator=g)
+    s = 0.005 + 0.01 * torch.rand((N, K // 64), device=dev, generator=g)
+    b = s * (3 * torch.rand((N, K // 64), device=dev, generator=g) - 9)
+    return w, s.bfloat16(), b.bfloat16()
+
+
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("M,K", [(15, 512), (15, 2048), (12, 4096), (15, 1536)])
+def test_few_rows_sum_as_exactly_as_one(dev, M, K, mean):
+    """Sharing the weights between rows costs no precision: the f32 sums of M
+    rows in one call are no further from 64 bits than the per-pair kernels'."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(K)
+    x = (torch.randn((M, K), device=dev, generator=g) + mean).bfloat16()
+    q = random_projection(g, dev, 32768, K)
+    together = sum_error(H.quantized_matmul(x, *q), x, *q)
+    single = sum_error(H.gather_qmm(x, *(t[None] for t in q),
+                                    torch.zeros(M, dtype=torch.int32, device=dev)), x, *q)
+    print(f"[qgemm] M={M} K={K} mean={mean}: {together:.2e}, one by one {single:.2e}", flush=True)
+    # some 40 outputs: the two rms have a spread of about 1 / sqrt(80) each
+    assert together <= 1.25 * single
 
 
 @pytest.mark.parametrize("dt,group", [(O.F16, 64), (O.BF16, 32), (O.BF16, 128)])
