@@ -42,12 +42,13 @@ struct GatherArgs {
 constexpr int64_t kGatherMinPairsPerExpert = 16;
 
 // bf16, group 64, 4 bits, x 16-byte aligned rows, w 16-byte aligned, K % 64,
-// the expert ids 16-byte aligned (read 4 at a time, the last up to 3 one by
-// one: a partly out-of-range 16-byte buffer load is not relied on) and under
-// 2 GiB.
+// the expert ids 16-byte aligned (read 4 at a time: a partly out-of-range
+// 16-byte buffer load is not relied on) and under 2 GiB. Pair counts that are
+// no multiple of 4 only where gather_ragged_fits.
 bool gather_grouped_supported(int dtype, int sdt, int group_size, int bits, const void* x,
                               int64_t xs, const void* w, int64_t k, const void* experts,
                               int64_t pairs);
+bool gather_ragged_fits(const GatherArgs& a);
 void gather_grouped_launch(const GatherArgs& a, hipStream_t s);
 // swiglu(gate, up) of the grouped regime in one launch (w/sc/bi: gate, w2/sc2/
 // bi2: up, same shapes); false where the fused kernel does not apply.

@@ -860,7 +860,7 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   __shared__ __align__(16) uint16_t xs[2][kGaBM][kQgPitch];
   __shared__ __align__(16) uint16_t wh[2][kHlBN][kQgPitch];
   __shared__ __align__(16) uint16_t wl[2][kHlBN][kQgPitch];
-  __shared__ int32_t list[kGaCap + 4];
+  __shared__ int32_t list[kGaCap];
   __shared__ int32_t cnt;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -891,11 +891,11 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   // the last pair read zeros and are never listed)
   static_assert(RND % 4 == 0, "whole 16-byte id loads");
   const __amdgpu_buffer_rsrc_t rid = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<void*>(a.experts), (short)0, (int)(a.pairs / 4 * 16), 0x00020000);
+      const_cast<void*>(a.experts), (short)0, (int)(a.pairs * 4), 0x00020000);
   int64_t scan = 0;
   while (scan < a.pairs) {
     // ---- fill the list from `scan` (stop before overflow)
-    const int rows = ga_list_phase<RND, true>(a, rid, e, scan, tid, &cnt, list);
+    const int rows = ga_list_phase<RND, false>(a, rid, e, scan, tid, &cnt, list);
 
     // ---- the listed pairs, kGaBM at a time, for each of this block's column tiles
     for (int nt = nt0; nt < nt1; ++nt)
@@ -1071,21 +1071,30 @@ constexpr int kXpBN = 64 * kXpWaves;  // columns per block pass
 // and waves 4-7 the up projection of the same 256 columns; after a pass the
 // up waves leave their bf16 results in LDS and the gate waves write
 // swiglu(gate, up), rounded as the reference's three calls round it.
-// GEN: any pair count, and the pairs split over gridDim.z blocks, `part` pairs
-// each. Its own form: the usual one (a multiple of 4, one part) keeps its
+// FORM: kXpUsual, a pair count that is a multiple of 4 in one part, keeps its
 // registers (with the last ids' code in it, it spilled 20 bytes and ran 1.5 %
-// slower).
-template <int RT, bool SW, bool GEN>
+// slower). kXpParts splits the pairs over gridDim.z blocks, `part` pairs each:
+// the same bits. kXpRagged does so for any pair count. Those calls took the
+// per-pair GEMV before, so their sums are to be no less exact: the codes as q
+// (expand_q, x in its own order) and scale and bias applied in f32 per group,
+// where 128 + q shows the rounding of sums that 128 Sx is still part of. Rms
+// error of outputs next to zero over the rms of all, 4099 pairs of 8 experts,
+// 2048 x 2048, x of unit deviation and mean 0 / 1: 1.3e-7 / 2.2e-7 here,
+// 4.8e-7 / 1.8e-6 per pair, 1.6e-6 at mean 0 with 128 + q. 20993 pairs of 128
+// experts, 512 -> 2048: 113.8 us, per pair 1313, with 128 + q 111.1.
+enum { kXpUsual = 0, kXpParts = 1, kXpRagged = 2 };
+template <int RT, bool SW, int FORM>
 __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t part) {
+  constexpr bool GEN = FORM != kXpUsual, RAG = FORM == kXpRagged;
   constexpr int BM = 16 * RT, NT = 4;
   constexpr int BNO = SW ? kXpBN / 2 : kXpBN;  // output columns per pass
   constexpr int XP = (BM * 8 + kXpT - 1) / kXpT;  // 16-byte x pieces per thread per group
   constexpr int RND = kGaRoundIds / kXpT;  // ids per thread per scan round
   __shared__ __align__(16) uint16_t xs[kXpXB][BM][kQgPitch];
-  __shared__ float sxs[8][BM];              // row sums, ring of 8 groups
+  __shared__ __align__(16) float sxs[8][BM];  // row sums, ring of 8 groups
   // scales and biases of 8 groups per column (double-buffered per 8 groups)
   __shared__ __align__(16) u32x4 ssb[2][kXpBN], bsb[2][kXpBN];
-  __shared__ int32_t list[kGaCap + (GEN ? 4 : 0)];
+  __shared__ int32_t list[kGaCap + (RAG ? 4 : 0)];
   __shared__ int32_t cnt;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1188,7 +1197,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
     for (int i = 0; i < XP; ++i) {
       const int c = tid + kXpT * i;
       if (c < BM * 8) {  // whole waves (BM * 8 is a multiple of 64)
-        *reinterpret_cast<u32x4*>(&xs[buf][c / 8][(c & 7) * 8]) = order_x4(q[i]);
+        *reinterpret_cast<u32x4*>(&xs[buf][c / 8][(c & 7) * 8]) = RAG ? q[i] : order_x4(q[i]);
         const float s8 = sum8_lanes(sum8_bf16(q[i]));
         if ((c & 7) == 0) sxs[g & 7][c / 8] = s8;
       }
@@ -1203,7 +1212,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
 
   while (scan < a.pairs) {
     // ---- list this expert's pairs from `scan` (stop before overflow)
-    const int rows = ga_list_phase<RND, GEN && !SW>(a, rid, e, scan, tid, &cnt, list);
+    const int rows = ga_list_phase<RND, RAG>(a, rid, e, scan, tid, &cnt, list);
 
     for (int nt = nt0; nt < nt1; ++nt)
     for (int t0 = 0; t0 < rows; t0 += BM) {
@@ -1228,14 +1237,15 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
       auto compute = [&](const u32x2_t (&q)[NT], int g) {
         const int sb = (g >> 3) & 1, j = g & 7;
         bf16x8_t bw[NT][2];
-        float sc[NT];
+        float sc[NT], bi[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           uint32_t w0 = q[t][0], w1 = q[t][1];
           asm volatile("" : "+v"(w0), "+v"(w1));
-          bw[t][0] = expand_codes_x4(w0, xm);
-          bw[t][1] = expand_codes_x4(w1, xm);
+          bw[t][0] = RAG ? expand_q(w0) : expand_codes_x4(w0, xm);
+          bw[t][1] = RAG ? expand_q(w1) : expand_codes_x4(w1, xm);
           sc[t] = stage_elem(ssb[sb], 64 * wave + 16 * t + l16, j);
+          if constexpr (RAG) bi[t] = stage_elem(bsb[sb], 64 * wave + 16 * t + l16, j);
         }
         const int buf = g & (kXpXB - 1);
 #pragma unroll
@@ -1255,6 +1265,13 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
             for (int t = 0; t < NT; ++t)
 #pragma unroll
               for (int r = 0; r < 4; ++r) acc[i][t][r] = __builtin_fmaf(sc[t], c[t][r], acc[i][t][r]);
+            if constexpr (RAG) {
+              const f32x4_t sx = *reinterpret_cast<const f32x4_t*>(&sxs[g & 7][i * 16 + 4 * lg]);
+#pragma unroll
+              for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][t][r] = __builtin_fmaf(bi[t], sx[r], acc[i][t][r]);
+            }
             // the row tile's update completes here (otherwise every MFMA
             // result of the group is held at once)
 #pragma unroll
@@ -1301,7 +1318,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
         for (int d = 0; d < 2; ++d) {
           const int g = g0 + d;
           compute(cw[d], g);
-          if ((g & 3) == 3) bias(g - 3);  // uniform
+          if (!RAG && (g & 3) == 3) bias(g - 3);  // uniform
           if ((g & 7) == 7) {
             // the next 8 groups' scales go to the other stage (its readers,
             // 8 groups back, are done); the 8 after that are requested
@@ -1480,10 +1497,22 @@ void gather_xp_launch(const GatherArgs& a, hipStream_t s) {
   }
   const int64_t part = ((a.pairs + gz - 1) / gz + 3) / 4 * 4;
   const dim3 grid((unsigned)gx, (unsigned)(a.E + 1), (unsigned)((a.pairs + part - 1) / part));
-  if (grid.z > 1 || a.pairs % 4 != 0)
-    HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, true>), grid, dim3(kXpT), 0, s, a, part);
+  if constexpr (!SW) {
+    if (a.pairs % 4 != 0) {
+      HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, kXpRagged>), grid, dim3(kXpT), 0, s, a, part);
+      return;
+    }
+  }
+  if (grid.z > 1)
+    HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, kXpParts>), grid, dim3(kXpT), 0, s, a, part);
   else
-    HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, false>), grid, dim3(kXpT), 0, s, a, part);
+    HGK_LAUNCH((gather_xp_kernel<HGK_XP_RT, SW, kXpUsual>), grid, dim3(kXpT), 0, s, a, part);
+}
+
+// A pair count that is no multiple of 4: where the per-pair GEMV has K, which
+// this form's sums are no less exact than (other K sum x (s q + b) per pair).
+bool gather_ragged_fits(const GatherArgs& a) {
+  return HGK_GATHER_XP && (a.K == 512 || a.K == 1024 || a.K == 2048 || a.K == 4096) && gather_xp_fits(a);
 }
 
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s) {

@@ -520,8 +520,10 @@ extern "C" int hgk_gather_qmm(int dtype, const void* x, int64_t x_rows, int64_t 
     g.sc = static_cast<const uint16_t*>(scales); g.bi = static_cast<const uint16_t*>(biases);
     g.experts = rhs_indices; g.experts_i32 = rhs_dtype == DT_I32; g.E = n_experts; g.N = n; g.K = k;
     g.pairs = pairs; g.y = static_cast<uint16_t*>(y); g.ys = y_row_stride;
-    gather_grouped_launch(g, s);
-    return launch_status(fn);
+    if (pairs % 4 == 0 || gather_ragged_fits(g)) {
+      gather_grouped_launch(g, s);
+      return launch_status(fn);
+    }
   }
   const bool vec_ok = dtype == DT_BF16 && aligned16(x) && x_row_stride % 8 == 0 && aligned16(w) &&
                       (reinterpret_cast<uintptr_t>(scales) & 1) == 0;

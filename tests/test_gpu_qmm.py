@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 import higgs_amd as H
 import oracle as O
@@ -295,6 +296,39 @@ def test_grouped_last_pairs_and_parts(dev, P, K):
     rows = np.unique(np.r_[0:5, 6:200, P // 2 - 70:P // 2 + 70, P - 300:P - 1])
     ref = O.gather_qmm(x, O.BF16, w, s, b, O.BF16, np.where(ex < 0, ex + E, ex)[rows], lhs=lhs[rows])
     _check(got[rows], ref, O.BF16, f"grouped P={P} K={K}")
+
+
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("P,K", [(4097, 512), (2050, 1024), (4099, 2048), (2051, 4096), (2049, 1536)])
+def test_ragged_pair_counts_sum_as_exactly_as_single_pairs(dev, P, K, mean):
+    """Pair counts that are no multiple of 4 came from the per-pair kernels to
+    the grouped one: its f32 sums are no further from 64 bits than theirs
+    (calls of fewer than 16 pairs per expert). Measured on the outputs within
+    1e-4 of the rms of all, whose bf16 rounding is below 1e-7 of it."""
+    E, N = 8, 2048
+    g = torch.Generator(device=dev)
+    g.manual_seed(K + P)
+    x = (torch.randn((P, K), device=dev, generator=g) + mean).bfloat16()
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, N, K // 8), dtype=torch.int32, device=dev, generator=g)
+    s = 0.005 + 0.01 * torch.rand((E, N, K // 64), device=dev, generator=g)
+    b = (s * (3 * torch.rand(s.shape, device=dev, generator=g) - 9)).bfloat16()
+    s = s.bfloat16()
+    ids = torch.randint(0, E, (P,), dtype=torch.int32, device=dev, generator=g)
+    grouped = H.gather_qmm(x, w, s, b, ids)
+    step = 16 * E - 4
+    single = torch.cat([H.gather_qmm(x[i:i + step], w, s, b, ids[i:i + step]) for i in range(0, P, step)])
+    ref = torch.empty((P, N), dtype=torch.float64, device=dev)
+    sh = torch.arange(0, 32, 4, device=dev, dtype=torch.int32)
+    for e in range(E):
+        q = ((w[e].unsqueeze(-1) >> sh) & 15).flatten(-2).double()
+        wd = q * s[e].double().repeat_interleave(64, -1) + b[e].double().repeat_interleave(64, -1)
+        ref[ids == e] = x[ids == e].double() @ wd.t()
+    rms = ref.pow(2).mean().sqrt()
+    near = ref.abs() < 1e-4 * rms
+    err = [float(((y.double() - ref)[near] / rms).pow(2).mean().sqrt()) for y in (grouped, single)]
+    print(f"[qmm] P={P} K={K} mean={mean}: grouped {err[0]:.2e}, single pairs {err[1]:.2e}", flush=True)
+    # more than 200 outputs: the two rms have a spread below 1 / 20 each
+    assert int(near.sum()) > 200 and err[0] <= 1.1 * err[1]
 
 
 # ------------------------------------------------------------------ fused gate/up/SwiGLU
