@@ -779,11 +779,17 @@ __device__ inline int64_t ga_row(const GatherArgs& a, int64_t p) {
 // fused gate + up + SwiGLU 327.2 -> 322.7 at the 4096-token Qwen3-Next MoE
 // prefill. The list order is free: every listed pair's output row is
 // computed on its own.
+// Whether another round fits is a decision of the whole block, since a round
+// holds a barrier: even rounds count their matches in one counter and odd ones
+// in another, and after a round's barrier every wave reads that round's, which
+// is next written two rounds, so a barrier, later. (Read from one counter of
+// all rounds, a fast wave's next matches could reach a slow wave before its
+// decision.)
 // Contains barriers: every thread of the block calls it. Returns the count.
 // Without TAIL the pair count must be a multiple of 4.
 template <int RND, bool TAIL>
 __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t rid, int64_t e,
-                                    int64_t& scan, int tid, int* cnt, int32_t* list) {
+                                    int64_t& scan, int tid, int (&cnt)[2], int32_t* list) {
   const int lane = tid & 63;
   // raw ids equal to e (and, for int32 ids, to e - E, which wraps to e)
   const uint32_t e1 = (uint32_t)e, e2 = a.experts_i32 ? (uint32_t)(e - a.E) : (uint32_t)e;
@@ -799,7 +805,8 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
       for (int k = 0; k < 4; ++k) r[4 * c + k] = v[k];
     }
   };
-  auto round = [&](const uint32_t (&ids)[RND]) {
+  int even = 0, odd = 0;  // matches listed in even and odd rounds (uniform)
+  auto round = [&](const uint32_t (&ids)[RND], int& counter, int& mine, int other) {
     const uint32_t p0 = (uint32_t)scan + RND * tid;
     // one ballot per id slot: a wave's matches are counted and placed with
     // scalar popcounts and mbcnt (no cross-lane prefix sum)
@@ -812,8 +819,8 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
     }
     if (tot > 0) {  // uniform per wave
       int base = 0;
-      if (lane == 0) base = atomicAdd(cnt, tot);
-      base = __builtin_amdgcn_readfirstlane(base);
+      if (lane == 0) base = atomicAdd(&counter, tot);
+      base = other + __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
       for (int i = 0; i < RND; ++i) {
         if (bal[i]) {  // uniform
@@ -826,28 +833,33 @@ __device__ inline int ga_list_phase(const GatherArgs& a, __amdgpu_buffer_rsrc_t 
     }
     scan += kGaRoundIds;
     __syncthreads();
+    mine = __builtin_amdgcn_readfirstlane(counter);
   };
   uint32_t ra[RND], rb[RND];
   load_round(ra, scan);
   __syncthreads();
-  if (tid == 0) *cnt = 0;
+  if (tid < 2) cnt[tid] = 0;
   __syncthreads();
+  bool last_even = false;
   while (scan < a.pairs) {
-    if (*cnt > kGaCap - kGaRoundIds) break;  // uniform: read after the round's barrier
+    if (even + odd > kGaCap - kGaRoundIds) break;
     load_round(rb, scan + kGaRoundIds);
-    round(ra);
-    if (scan >= a.pairs || *cnt > kGaCap - kGaRoundIds) break;
+    round(ra, cnt[0], even, odd);
+    last_even = scan >= a.pairs || even + odd > kGaCap - kGaRoundIds;
+    if (last_even) break;
     load_round(ra, scan + kGaRoundIds);
-    round(rb);
+    round(rb, cnt[1], odd, even);
   }
   if (tail && scan >= a.pairs) {  // uniform; the list has room for 3 more
+    int& counter = cnt[last_even ? 1 : 0];
     if (tid < (int)tail) {
       const uint32_t id = reinterpret_cast<const uint32_t*>(a.experts)[pairs + tid];
-      if (id == e1 || id == e2) list[atomicAdd(cnt, 1)] = (int32_t)(pairs + tid);
+      if (id == e1 || id == e2) list[atomicAdd(&counter, 1) + (last_even ? even : odd)] = (int32_t)(pairs + tid);
     }
     __syncthreads();
+    (last_even ? odd : even) = __builtin_amdgcn_readfirstlane(counter);
   }
-  return *cnt;
+  return even + odd;
 }
 
 template <int WAVES>
@@ -861,7 +873,7 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   __shared__ __align__(16) uint16_t wh[2][kHlBN][kQgPitch];
   __shared__ __align__(16) uint16_t wl[2][kHlBN][kQgPitch];
   __shared__ int32_t list[kGaCap];
-  __shared__ int32_t cnt;
+  __shared__ int cnt[2];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -895,7 +907,7 @@ __global__ __launch_bounds__(WAVES * 64) void gather_hl_kernel(GatherArgs a) {
   int64_t scan = 0;
   while (scan < a.pairs) {
     // ---- fill the list from `scan` (stop before overflow)
-    const int rows = ga_list_phase<RND, false>(a, rid, e, scan, tid, &cnt, list);
+    const int rows = ga_list_phase<RND, false>(a, rid, e, scan, tid, cnt, list);
 
     // ---- the listed pairs, kGaBM at a time, for each of this block's column tiles
     for (int nt = nt0; nt < nt1; ++nt)
@@ -1081,7 +1093,7 @@ constexpr int kXpBN = 64 * kXpWaves;  // columns per block pass
 // error of outputs next to zero over the rms of all, 4099 pairs of 8 experts,
 // 2048 x 2048, x of unit deviation and mean 0 / 1: 1.3e-7 / 2.2e-7 here,
 // 4.8e-7 / 1.8e-6 per pair, 1.6e-6 at mean 0 with 128 + q. 20993 pairs of 128
-// experts, 512 -> 2048: 113.8 us, per pair 1313, with 128 + q 111.1.
+// experts, 512 -> 2048: 119 us, per pair 1313, with 128 + q 111.
 enum { kXpUsual = 0, kXpParts = 1, kXpRagged = 2 };
 template <int RT, bool SW, int FORM>
 __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t part) {
@@ -1095,7 +1107,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
   // scales and biases of 8 groups per column (double-buffered per 8 groups)
   __shared__ __align__(16) u32x4 ssb[2][kXpBN], bsb[2][kXpBN];
   __shared__ int32_t list[kGaCap + (RAG ? 4 : 0)];
-  __shared__ int32_t cnt;
+  __shared__ int cnt[2];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1212,7 +1224,7 @@ __global__ __launch_bounds__(kXpT) void gather_xp_kernel(GatherArgs a, int64_t p
 
   while (scan < a.pairs) {
     // ---- list this expert's pairs from `scan` (stop before overflow)
-    const int rows = ga_list_phase<RND, RAG>(a, rid, e, scan, tid, &cnt, list);
+    const int rows = ga_list_phase<RND, RAG>(a, rid, e, scan, tid, cnt, list);
 
     for (int nt = nt0; nt < nt1; ++nt)
     for (int t0 = 0; t0 < rows; t0 += BM) {

@@ -298,6 +298,26 @@ def test_grouped_last_pairs_and_parts(dev, P, K):
     _check(got[rows], ref, O.BF16, f"grouped P={P} K={K}")
 
 
+@pytest.mark.parametrize("P,K", [(20000, 512), (20002, 512), (16384, 576)],
+                         ids=["parts", "ragged", "other-K"])
+def test_grouped_list_that_fills_again_and_again(dev, P, K):
+    """Nearly all pairs on one expert of two, so that a block's list of pairs
+    fills, is drained and fills again: every pair is computed once, to the bits
+    of the other pairs with the same row and expert."""
+    R, E, N = 37, 2, 72
+    x, w, s, b, ex = _case(2541 + P, P, R, E, N, K)
+    ex = np.ones_like(ex)
+    ex[::997] = 0
+    lhs = (np.arange(P) % R).astype(np.int32)
+    got = _run(dev, x, w, s, b, ex, O.BF16, lhs=lhs)
+    want = O.gather_qmm(x, O.BF16, w, s, b, O.BF16, np.repeat([0, 1], R).astype(np.int32),
+                        lhs=np.tile(np.arange(R), 2).astype(np.int32)).reshape(2, R, N)
+    one = np.stack([[got[np.flatnonzero((ex == e) & (lhs == r))[0]] if ((ex == e) & (lhs == r)).any()
+                     else want[e, r] for r in range(R)] for e in (0, 1)])
+    _check(one, want, O.BF16, f"long list P={P} K={K}")
+    assert np.array_equal(got, one[ex, lhs])
+
+
 @pytest.mark.parametrize("mean", [0.0, 1.0])
 @pytest.mark.parametrize("P,K", [(4097, 512), (2050, 1024), (4099, 2048), (2051, 4096), (2049, 1536)])
 def test_ragged_pair_counts_sum_as_exactly_as_single_pairs(dev, P, K, mean):
