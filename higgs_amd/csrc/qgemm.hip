@@ -1528,7 +1528,8 @@ bool gather_ragged_fits(const GatherArgs& a) {
 }
 
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s) {
-  if (!HGK_GATHER_XP || !gather_xp_fits(a) || !a.w2 || !a.sc2 || !a.bi2 ||
+  // (the fused kernel reads the ids 4 at a time only)
+  if (!HGK_GATHER_XP || !gather_xp_fits(a) || a.pairs % 4 != 0 || !a.w2 || !a.sc2 || !a.bi2 ||
       (reinterpret_cast<uintptr_t>(a.w2) & 15) != 0)
     return false;
   gather_xp_launch<true>(a, s);

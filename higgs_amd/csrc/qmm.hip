@@ -632,7 +632,7 @@ extern "C" int hgk_gather_qmm_swiglu(int dtype, const void* x, int64_t x_rows,
   if (pairs >= kGatherMinPairsPerExpert * n_experts) {
     // many pairs per expert (prefill): the grouped matrix-core kernel's fused
     // form, where it applies
-    if (pairs > 0 && pairs % 4 == 0 && n_experts < 65535 &&
+    if (pairs > 0 && n_experts < 65535 &&
         gather_grouped_supported(dtype, scales_dtype, group_size, bits, x, x_row_stride, w_gate, k,
                                  rhs_indices, pairs)) {
       GatherArgs g{};

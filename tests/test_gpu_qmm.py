@@ -476,6 +476,20 @@ def test_fused_gate_up_swiglu_grouped_prefill(dev):
         assert np.array_equal(got4, O.glu(O.ACT_SILU, gh4, uh4, O.BF16)), f"N={N4}"
 
 
+@pytest.mark.parametrize("T", [257, 258, 259])
+def test_fused_gate_up_swiglu_of_ragged_pair_counts(dev, T):
+    """Prefill-sized pair counts that are no multiple of 4: the fused kernel does
+    not take them and the three calls give their result, the last pairs too."""
+    E, N, K = 4, 64, 512
+    x, g, u, ex = _fused_case(4301 + T, T, 1, E, N, K)
+    got = to_host(_fused_dev(dev, x, g, u, ex, 1))
+    d = lambda t: to_dev(t, O.BF16, dev)
+    gh, uh = (to_host(H.gather_qmm(d(x), words_dev(m[0], dev), d(m[1]), d(m[2]), to_dev(ex, O.I32, dev)))
+              for m in (g, u))
+    assert np.array_equal(got, O.glu(O.ACT_SILU, gh, uh, O.BF16))
+    _check(gh, O.gather_qmm(x, O.BF16, *g, O.BF16, ex), O.BF16, f"ragged T={T}: gate")
+
+
 def test_fused_gate_up_swiglu_routing_and_fallback(dev):
     """Out-of-range experts give zero rows, as the three calls do; in the
     grouped (prefill) regime the fused entry runs the grouped kernel's fused
