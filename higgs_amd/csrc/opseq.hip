@@ -716,15 +716,25 @@ void make_chains(DevOpList* L) {
     } else {
       DevOp& q = L->ops[p];
       q.next = i;
-      const bool carry = d.kind == kOpAddRms && q.kind == kOpAddRms && q.h && d.x == q.h &&
+      bool carry = d.kind == kOpAddRms && q.kind == kOpAddRms && q.h && d.x == q.h &&
                          d.x_tok == q.h_tok && d.x_row == q.h_row && d.rows == q.rows && d.n == q.n &&
                          d.rows * d.g <= kOpThreads;
+      // where q's y lies on its h, x is y, stored last
+      int64_t over = INT64_MAX;
+      if (carry)
+        for (const Range& a : rg[p])
+          for (const Range& b : rg[p])
+            if (a.write && b.write && &a < &b) over = std::min(over, first_overlap(a, b));
+      carry = carry && over > 0;
       // (d.next names the op whose h is carried until the chain's next op is known)
       d.next = p;
       bool wait = false;
       for (int k = since[c]; k < i && !wait; ++k) wait = chain[k] == c && conflict(k, i, carry) == 0;
       d.next = INT32_MAX;
-      if (carry && !wait) d.flags = kOpCarry;
+      if (carry && !wait) {
+        d.flags = kOpCarry;
+        safe = std::min(safe, over);
+      }
       if (wait) {
         d.flags |= kOpWait;
         since[c] = i;

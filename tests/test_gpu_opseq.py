@@ -232,6 +232,29 @@ def test_dependent_ops_over_shared_buffers(dev, seed):
             assert np.array_equal(to_host(got), to_host(want)), f"buffer {i}"
 
 
+@pytest.mark.parametrize("n", [64, 2048])
+def test_a_norm_written_over_its_residual(dev, n):
+    """y on the address of h: y is stored last, so the next op reads y, whether
+    or not it could have taken h from registers."""
+    T, dt = 5, torch.bfloat16
+    g = torch.Generator(device=dev)
+    g.manual_seed(n)
+    x, r1, r2, r3 = (torch.randn(T, n, generator=g, device=dev).to(dt) for _ in range(4))
+    w = torch.randn(n, generator=g, device=dev).to(dt)
+    a, h2, y2, h3, y3 = (torch.zeros(T, n, dtype=dt, device=dev) for _ in range(5))
+    seq = H.OpSequence(dt, torch.device(dev))
+    seq.add_rms_norm(x, r1, w, 1e-6, a, a)
+    seq.add_rms_norm(a, r2, w, 1e-6, y2, h2)
+    seq.add_rms_norm(h2, r3, w, 1e-6, y3, h3)
+    seq.run(T)
+    _, y1 = H.add_rms_norm(x, r1, w, 1e-6)
+    want2 = H.add_rms_norm(y1, r2, w, 1e-6)
+    want3 = H.add_rms_norm(want2[0], r3, w, 1e-6)
+    for what, got, want in (("y1", a, y1), ("h2", h2, want2[0]), ("y2", y2, want2[1]),
+                            ("h3", h3, want3[0]), ("y3", y3, want3[1])):
+        _same_bits(got, want, what)
+
+
 def test_buffers_that_meet_at_a_later_token(dev):
     """Two ops whose outputs share bytes only from some token on (views with
     different token strides): up to there they run side by side, over more
