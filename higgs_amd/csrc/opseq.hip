@@ -39,7 +39,12 @@
 // The op list is a device array written by hgk_op_list_upload into memory the
 // caller owns; this file allocates nothing.
 #include <algorithm>
+#include <array>
 #include <cmath>
+#include <iterator>
+#include <map>
+#include <new>
+#include <utility>
 #include <vector>
 
 #include "../../include/higgs_hip.h"
@@ -603,10 +608,13 @@ bool same_positions(const DevOp& p, const DevOp& d) {
 }
 
 // The bytes an op reads or writes for token t: [lo + t tok, lo + t tok + span).
+// key: who touches them, where one thread holds one 16-byte unit (add + norm
+// over at most kOpThreads units): equal keys, the same threads. -1: others.
 struct Range {
   int64_t lo, span, tok;
   bool write;
-  int64_t row;  // row stride where one thread holds one 16-byte unit (add + norm), else -1
+  int op, key;
+  int64_t end() const { return lo + span; }
 };
 
 // The smallest t >= 0 for which a's and b's bytes of token t overlap.
@@ -620,90 +628,175 @@ int64_t first_overlap(Range a, Range b) {
   return d0 + t * dt < a.span ? t : INT64_MAX;
 }
 
-std::vector<Range> op_ranges(const DevOp& d) {
+// An op's ranges; range 0 is x.
+std::vector<Range> op_ranges(const DevOp& d, int op, std::map<std::array<int64_t, 5>, int>& keys) {
   std::vector<Range> v;
   const bool own = d.kind == kOpAddRms && d.rows * d.g <= kOpThreads;
   auto add = [&](const void* p, int64_t tok, int64_t rows, int64_t row, bool write) {
-    if (p && rows > 0) v.push_back({(int64_t)(intptr_t)p, ((rows - 1) * row + d.n) * 2, tok * 2, write, own ? row : -1});
+    if (!p || rows <= 0) return;
+    const int64_t lo = (int64_t)(intptr_t)p;
+    int key = -1;
+    if (own) key = keys.try_emplace({lo, tok, row, rows, d.n}, (int)keys.size()).first->second;
+    v.push_back({lo, ((rows - 1) * row + d.n) * 2, tok * 2, write, op, key});
+  };
+  auto other = [&](const void* p, int64_t off, int64_t bytes, int64_t tok) {
+    v.push_back({(int64_t)(intptr_t)p + off, bytes, tok, false, op, -1});
   };
   add(d.x, d.x_tok, d.rows, d.x_row, false);
   add(d.y, d.y_tok, d.rows, d.y_row, true);
-  if (d.w) v.push_back({(int64_t)(intptr_t)d.w, d.n * 2, 0, false, -1});
+  if (d.w) other(d.w, 0, d.n * 2, 0);
   if (d.kind == kOpAddRms || d.kind == kOpGlu) add(d.r, d.r_tok, d.rows, d.r_row, false);
   if (d.kind == kOpAddRms) add(d.h, d.h_tok, d.rows, d.h_row, true);
   if (d.kind == kOpGated) {
     const int64_t groups = (d.rows + d.zg - 1) / d.zg, rows = std::min<int64_t>(d.rows, d.zg);
     const int64_t far = (groups - 1) * d.zgs;  // may be negative
     const int64_t lo = std::min<int64_t>(far, 0), hi = std::max<int64_t>(far, 0) + (rows - 1) * d.r_row + d.n;
-    v.push_back({(int64_t)(intptr_t)d.r + lo * 2, (hi - lo) * 2, d.r_tok * 2, false, -1});
+    other(d.r, lo * 2, (hi - lo) * 2, d.r_tok * 2);
   }
   if (d.kind == kOpRope) {
     add(d.r, d.r_tok, d.k_rows, d.r_row, false);
     add(d.h, d.h_tok, d.k_rows, d.h_row, true);
-    add(d.w2, 0, 1, 0, false);
-    if (d.offsets) v.push_back({(int64_t)(intptr_t)d.offsets, 4, 4, false, -1});
+    if (d.w2) other(d.w2, 0, d.n * 2, 0);
+    if (d.offsets) other(d.offsets, 0, 4, 4);
   }
   return v;
 }
 
+struct Groups {
+  std::vector<int> root, size;
+  explicit Groups(int n) : root(n), size(n, 1) {
+    for (int i = 0; i < n; ++i) root[i] = i;
+  }
+  int find(int i) {
+    while (root[i] != i) i = root[i] = root[root[i]];
+    return i;
+  }
+  void join(int i, int j) {
+    i = find(i);
+    j = find(j);
+    if (i == j) return;
+    size[j] += size[i];
+    root[i] = j;
+  }
+};
+
+// Join the ops that share bytes of token 0, one of them writing: a sweep over
+// the ranges by address. Of the writes that reach the current address one
+// stands for all (they overlap there, so their ops are joined; the one that
+// ends last is met by whatever meets any), and so does one of the reads that a
+// write has joined.
+void join_overlaps(std::vector<Range> all, Groups& g) {
+  std::sort(all.begin(), all.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
+  Range w{};  // the write that ends last (op -1: none)
+  w.op = -1;
+  std::vector<Range> reads;  // not joined with each other; some have ended
+  for (const Range& r : all) {
+    if (w.op >= 0 && w.end() > r.lo) g.join(w.op, r.op);
+    if (!r.write) {
+      reads.push_back(r);
+      continue;
+    }
+    Range last = r;
+    for (const Range& q : reads) {
+      if (q.end() <= r.lo) continue;
+      g.join(q.op, r.op);
+      if (q.end() > last.end()) last = q;
+    }
+    reads.clear();
+    if (last.op != r.op || last.end() > r.end()) reads.push_back(last);
+    if (w.op < 0 || w.end() <= r.lo || r.end() > w.end()) w = r;
+  }
+}
+
+// The first token t >= 1 for which ops share bytes, one of them writing, that
+// they do not share for token 0 (only ranges with different token strides do),
+// or `safe` where that is smaller. Per pair of strides, each range of the
+// larger one meets the ranges above it, nearest first, until a range is too far
+// to be met before `safe`.
+int64_t first_later_overlap(const std::vector<Range>& all, int64_t safe) {
+  std::map<int64_t, std::array<std::vector<Range>, 2>> by;  // per stride: all ranges, the writes
+  for (const Range& r : all) {
+    by[r.tok][0].push_back(r);
+    if (r.write) by[r.tok][1].push_back(r);
+  }
+  // (many strides would make many pairs: such a list runs in order)
+  if (by.size() > 32) return 0;
+  for (auto& [tok, lists] : by)
+    for (auto& l : lists) std::sort(l.begin(), l.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
+  for (const auto& [small, as] : by)
+    for (const auto& [large, bs] : by) {
+      if (large <= small) continue;
+      for (const Range& b : bs[0]) {
+        const std::vector<Range>& l = as[b.write ? 0 : 1];
+        auto a = std::lower_bound(l.begin(), l.end(), b.end(), [](const Range& r, int64_t end) { return r.lo < end; });
+        for (; a != l.end() && (a->lo - b.end()) / (large - small) + 1 < safe; ++a)
+          if (a->op != b.op) safe = std::min(safe, first_overlap(*a, b));
+      }
+    }
+  return safe;
+}
+
+// The bytes that a chain's ops have read (written) since its last wait, as
+// disjoint segments; a segment has the key of its only range, or -1.
+struct Touched {
+  std::map<int64_t, std::pair<int64_t, int>> seg;  // lo -> end, key
+  // whether [r.lo, r.end()) meets a segment, other than one of key `but` (>= 0)
+  bool meets(const Range& r, int but) const {
+    auto it = seg.upper_bound(r.lo);
+    if (it != seg.begin() && std::prev(it)->second.first > r.lo) --it;
+    for (; it != seg.end() && it->first < r.end(); ++it)
+      if (but < 0 || it->second.second != but) return true;
+    return false;
+  }
+  void add(const Range& r) {
+    int64_t lo = r.lo, end = r.end();
+    int key = r.key;
+    auto it = seg.upper_bound(lo);
+    if (it != seg.begin() && std::prev(it)->second.first > lo) --it;
+    while (it != seg.end() && it->first < end) {
+      if (it->second.second != key) key = -1;
+      lo = std::min(lo, it->first);
+      end = std::max(end, it->second.first);
+      it = seg.erase(it);
+    }
+    seg.emplace(lo, std::make_pair(end, key));
+  }
+};
+
 // Sort the list's ops into chains (see the top of the file).
 void make_chains(DevOpList* L) {
   const int n = L->count;
+  std::map<std::array<int64_t, 5>, int> keys;
   std::vector<std::vector<Range>> rg(n);
-  for (int i = 0; i < n; ++i) rg[i] = op_ranges(L->ops[i]);
-  // The first token for which ops i < j conflict. carry: for j as a carried op
-  // (its x, range 0, is in registers), and where j writes exactly what i read or
-  // wrote, by the same threads (rows of the same shape), program order is enough.
-  auto conflict = [&](int i, int j, bool carry) {
-    const bool same = L->ops[i].rows == L->ops[j].rows && L->ops[i].n == L->ops[j].n;
-    int64_t t = INT64_MAX;
-    for (const Range& a : rg[i])
-      for (const Range& b : rg[j]) {
-        if (!a.write && !b.write) continue;
-        const bool layout = same && a.row >= 0 && a.row == b.row && a.lo == b.lo && a.tok == b.tok;
-        if (carry && layout && (b.write || (&b == &rg[j][0] && i == L->ops[j].next))) continue;
-        t = std::min(t, first_overlap(a, b));
-      }
-    return t;
-  };
-  std::vector<int> root(n), size(n, 1), chain(n);
-  for (int i = 0; i < n; ++i) root[i] = i;
-  auto find = [&](int i) {
-    while (root[i] != i) i = root[i] = root[root[i]];
-    return i;
-  };
-  int64_t safe = INT32_MAX;
-  for (int j = 0; j < n; ++j)
-    for (int i = 0; i < j; ++i) {
-      const int64_t t = conflict(i, j, false);
-      if (t > 0) {
-        safe = std::min(safe, t);
-      } else if (find(i) != find(j)) {
-        size[find(j)] += size[find(i)];
-        root[find(i)] = find(j);
-      }
-    }
+  std::vector<Range> all;
+  for (int i = 0; i < n; ++i) {
+    rg[i] = op_ranges(L->ops[i], i, keys);
+    all.insert(all.end(), rg[i].begin(), rg[i].end());
+  }
+  Groups groups(n);
+  join_overlaps(all, groups);
+  int64_t safe = first_later_overlap(all, INT32_MAX);
   // the largest group of dependent ops is chain 0; each other group goes to
   // the chain with the fewest ops so far
   int big = 0;
   for (int i = 0; i < n; ++i)
-    if (size[find(i)] > size[find(big)]) big = i;
-  std::vector<int> of(n, -1);
+    if (groups.size[groups.find(i)] > groups.size[groups.find(big)]) big = i;
+  std::vector<int> of(n, -1), chain(n);
   int load[kChains] = {};
-  of[find(big)] = 0;
-  load[0] = size[find(big)];
+  of[groups.find(big)] = 0;
+  load[0] = groups.size[groups.find(big)];
   for (int i = 0; i < n; ++i) {
-    int& c = of[find(i)];
+    int& c = of[groups.find(i)];
     if (c < 0) {
       c = (int)(std::min_element(load, load + kChains) - load);
-      load[c] += size[find(i)];
+      load[c] += groups.size[groups.find(i)];
     }
     chain[i] = c;
   }
-  int last[kChains], since[kChains], rope[kChains];
+  int last[kChains], rope[kChains];
+  Touched reads[kChains], writes[kChains];
   for (int c = 0; c < kChains; ++c) {
     last[c] = rope[c] = -1;
-    since[c] = 0;  // first op after the chain's last wait
     if (c < n) L->ops[c].first = INT32_MAX;
   }
   for (int i = 0; i < n; ++i) {
@@ -717,8 +810,8 @@ void make_chains(DevOpList* L) {
       DevOp& q = L->ops[p];
       q.next = i;
       bool carry = d.kind == kOpAddRms && q.kind == kOpAddRms && q.h && d.x == q.h &&
-                         d.x_tok == q.h_tok && d.x_row == q.h_row && d.rows == q.rows && d.n == q.n &&
-                         d.rows * d.g <= kOpThreads;
+                   d.x_tok == q.h_tok && d.x_row == q.h_row && d.rows == q.rows && d.n == q.n &&
+                   d.rows * d.g <= kOpThreads;
       // where q's y lies on its h, x is y, stored last
       int64_t over = INT64_MAX;
       if (carry)
@@ -726,20 +819,24 @@ void make_chains(DevOpList* L) {
           for (const Range& b : rg[p])
             if (a.write && b.write && &a < &b) over = std::min(over, first_overlap(a, b));
       carry = carry && over > 0;
-      // (d.next names the op whose h is carried until the chain's next op is known)
-      d.next = p;
+      // a carried op reads x from registers, and where it writes what the same
+      // threads read or wrote before, program order is enough
       bool wait = false;
-      for (int k = since[c]; k < i && !wait; ++k) wait = chain[k] == c && conflict(k, i, carry) == 0;
-      d.next = INT32_MAX;
+      for (size_t k = carry ? 1 : 0; k < rg[i].size() && !wait; ++k) {
+        const Range& r = rg[i][k];
+        const int but = carry && r.write ? r.key : -1;
+        wait = writes[c].meets(r, but) || (r.write && reads[c].meets(r, but));
+      }
       if (carry && !wait) {
         d.flags = kOpCarry;
         safe = std::min(safe, over);
       }
       if (wait) {
         d.flags |= kOpWait;
-        since[c] = i;
+        reads[c] = writes[c] = Touched();
       }
     }
+    for (const Range& r : rg[i]) (r.write ? writes : reads)[c].add(r);
     last[c] = i;
     if (d.kind == kOpRope) {
       if (rope[c] >= 0 && same_positions(L->ops[rope[c]], d)) d.same_table |= 2;
@@ -760,7 +857,7 @@ extern "C" int64_t hgk_op_list_bytes(int n_ops) {
 }
 
 extern "C" int hgk_op_list_upload(int dtype, const hgk_op* ops, int n_ops, void* dev_list,
-                                  int64_t dev_bytes, void* stream) {
+                                  int64_t dev_bytes, void* stream) try {
   clear_error();
   const char* fn = "hgk_op_list_upload";
   if (dtype != DT_BF16 && dtype != DT_F16)
@@ -794,6 +891,8 @@ extern "C" int hgk_op_list_upload(int dtype, const hgk_op* ops, int n_ops, void*
   if (e == hipSuccess) e = hipStreamSynchronize(as_stream(stream));
   if (e != hipSuccess) return fail(HGK_ERR_HIP, "%s: copy failed: %s", fn, hipGetErrorString(e));
   return HGK_OK;
+} catch (const std::bad_alloc&) {
+  return fail(HGK_ERR_HIP, "hgk_op_list_upload: out of host memory");
 }
 
 extern "C" int hgk_op_list_run(int dtype, const void* dev_list, int n_ops, int64_t tokens,

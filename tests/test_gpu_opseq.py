@@ -11,6 +11,8 @@ in_proj_qkvz) or q/k RMSNorm + partial RoPE (every fourth layer, q the first
 projections' outputs are random stand-ins."""
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -174,31 +176,45 @@ def test_op_sequence_fewer_tokens_and_a_foreign_list(dev):
         _same_bits(v, before[k], f"foreign list {k}")
 
 
-@pytest.mark.parametrize("seed", range(6))
+@pytest.mark.parametrize("seed", range(10))
 def test_dependent_ops_over_shared_buffers(dev, seed):
-    """Random lists over a small pool of buffers, so that ops read, overwrite
-    and re-read each other's results (in place, through column slices and
-    through views with another token stride), against the separate calls bit
-    for bit. Chains of dependent ops run in order whatever else runs beside."""
+    """Random lists of all five kinds of op over a small pool of buffers, so that
+    ops read, overwrite and re-read each other's results (in place, through
+    column slices and, in every other list, with views of two token strides),
+    against the separate calls bit for bit. Chains of dependent ops run in order
+    whatever else runs beside."""
     T, n, dt = 5, 256, torch.bfloat16
     r = np.random.default_rng(100 + seed)
     g = torch.Generator(device=dev)
     g.manual_seed(seed)
     w = torch.randn(n, generator=g, device=dev).to(dt)
-    base = [torch.randn(T, 2 * n, generator=g, device=dev).to(dt) for _ in range(5)]
+    wh = torch.randn(64, generator=g, device=dev).to(dt)
+    offsets = torch.randint(0, 99, (T,), dtype=torch.int32, device=dev, generator=g)
+    base = [torch.randn(3 * T, 2 * n, generator=g, device=dev).to(dt) for _ in range(5)]
     start = [b.clone() for b in base]
 
-    def view(pool, i, half):  # [T, n]: one half of buffer i's rows
-        return pool[i][:, half * n:(half + 1) * n]
+    def view(pool, i, half, rows):  # [T, n]: one half of buffer i's rows 0, 1, .. or T, T + 2, ..
+        return (pool[i][T::2] if rows else pool[i])[:T, half * n:(half + 1) * n]
 
+    def heads(v):  # [T, 4, 64]
+        return v.unflatten(-1, (4, 64))
+
+    # (the views of one buffer have one stride: where two meet, it is for different tokens, whose
+    # order no list defines)
+    two = seed % 2 == 1
+    at = lambda i: int(two and i >= 3)
+    pick = lambda: (lambda i: (i, int(r.integers(2)), at(i)))(int(r.integers(5)))
     ops, carry = [], None
     for _ in range(40):
-        kind = r.choice(["add", "add", "add", "rms", "glu"])
-        a, b, c, d = [(int(r.integers(5)), int(r.integers(2))) for _ in range(4)]
+        kind = r.choice(["add", "add", "add", "rms", "glu", "gated", "rope"])
+        a, b, c, d = pick(), pick(), pick(), pick()
         if kind == "add" and carry is not None and r.random() < 0.7:
             a = carry  # the residual stream, sometimes updated in place
             d = a if r.random() < 0.3 else d
-        if c == d or (kind == "add" and c in (a, b)):
+        if kind == "rope":
+            if len({a, b, c, d}) < 4:
+                continue
+        elif c == d or (kind in ("add", "gated") and c in (a, b)):
             continue
         if kind == "add" and d == b:
             continue
@@ -211,25 +227,63 @@ def test_dependent_ops_over_shared_buffers(dev, seed):
             seq.add_rms_norm(x, y, w, 1e-6, out, h)
         elif kind == "rms":
             seq.rms_norm(x, w, 1e-6, out)
+        elif kind == "gated":
+            seq.gated_rms_norm(heads(x), heads(y), wh, 1e-6, heads(out))
+        elif kind == "rope":
+            # (two tables in turn: a chain's ops reuse one only where it is theirs)
+            seq.qk_norm_rope(heads(x), heads(y), wh, wh, 1e-6, 32, 1e4 if a[1] else 1e6, heads(out),
+                             heads(h), offsets=offsets)
         else:
             seq.glu(ACT_SILU, x, y, out)
     ref = [b.clone() for b in start]
     for kind, a, b, c, d in ops:
         x, y, out, h = (view(ref, *p) for p in (a, b, c, d))
+        x, y = x.contiguous(), y.contiguous()
         if kind == "add":
-            hh, yy = H.add_rms_norm(x.contiguous(), y.contiguous(), w, 1e-6)
+            hh, yy = H.add_rms_norm(x, y, w, 1e-6)
             h.copy_(hh)
             out.copy_(yy)
         elif kind == "rms":
-            out.copy_(H.rms_norm(x.contiguous(), w, 1e-6))
+            out.copy_(H.rms_norm(x, w, 1e-6))
+        elif kind == "gated":
+            out.copy_(H.gated_rms_norm(heads(x), heads(y), wh, 1e-6).flatten(1))
+        elif kind == "rope":
+            q, k = H.qk_norm_rope(heads(x).unsqueeze(1), heads(y).unsqueeze(1), wh, wh, 1e-6, 32,
+                                  1e4 if a[1] else 1e6, 1.0, 0, offsets=offsets)
+            out.copy_(q[:, :, 0].flatten(1))
+            h.copy_(k[:, :, 0].flatten(1))
         else:
-            out.copy_(H.swiglu(x.contiguous(), y.contiguous()))
+            out.copy_(H.swiglu(x, y))
     for _ in range(2):  # the same list again, from the same start
         for b, s in zip(base, start):
             b.copy_(s)
         seq.run(T)
         for i, (got, want) in enumerate(zip(base, ref)):
             assert np.array_equal(to_host(got), to_host(want)), f"buffer {i}"
+
+
+def test_a_long_list_uploads_in_proportion(dev):
+    """Sorting a list into chains takes time in proportion to its length: 4096
+    ops (the most a list holds) upload in at most 24 times the time of 512, the
+    least of three times each (8 times the ops; pairs of ops: 64)."""
+    T, n, dt = 2, 64, torch.bfloat16
+    x = torch.zeros(T, n, dtype=dt, device=dev)
+    pool = torch.zeros(3 * 4096, T, n, dtype=dt, device=dev)
+    w = torch.ones(n, dtype=dt, device=dev)
+    least = {}
+    for n_ops in (512, 4096):
+        seq, h = H.OpSequence(dt, torch.device(dev)), x
+        for i in range(n_ops):
+            seq.add_rms_norm(h, pool[3 * i], w, 1e-6, pool[3 * i + 1], pool[3 * i + 2])
+            h = pool[3 * i + 2]
+        times = []
+        for _ in range(3):
+            t0 = time.perf_counter()
+            seq.upload()
+            times.append(time.perf_counter() - t0)
+        least[n_ops] = min(times)
+    print(f"[opseq] upload: 512 ops {least[512] * 1e3:.2f} ms, 4096 {least[4096] * 1e3:.2f} ms", flush=True)
+    assert least[4096] <= 24 * least[512]
 
 
 @pytest.mark.parametrize("n", [64, 2048])
