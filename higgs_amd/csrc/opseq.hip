@@ -16,15 +16,19 @@
 //
 // Most of those ops do not depend on each other: of the 192 ops of a 48-layer
 // Qwen3-Next step, 96 form the residual chain and 96 read nothing that the
-// list writes. Upload therefore sorts the ops into chains (ops that share a
-// buffer, one of them writing it, for the same token stay in one chain, in
-// list order), and a token gets kChains workgroups, one per chain. Within a
+// list writes. Upload therefore sorts the ops into up to kChains chains (ops
+// that share a buffer, one of them writing it, for the same token stay in one
+// chain, in list order), and a token gets a workgroup per chain where there are
+// few tokens, else fewer that walk several chains each. Within a
 // chain an op waits for earlier stores (a wait on every outstanding memory
 // operation, then the workgroup barrier) only where it touches what an op
 // since the last wait wrote, and a run of residual adds + norms over the same
 // rows carries h in registers, with the next residual and weight loaded
-// beside the current sum. 64 tokens x 48 layers: 466 us with every op in one
-// workgroup, waiting; 159 with chains.
+// beside the current sum. 64 tokens x 48 layers, every buffer in cache: 411 us
+// with every op in one workgroup, waiting; 125 with chains (buffers that change
+// between runs: 466 and 159). What the launch then measures is the list's own
+// dependences: a model that fills the list's inputs from the list's outputs
+// (attention, experts) cannot run the whole step in one launch.
 // Every consumer of an op's output inside the launch is the same workgroup,
 // so workgroup-scope ordering is all the data needs; other consumers see it
 // after the launch. Buffers that only meet for some later token (views with
@@ -57,7 +61,7 @@ namespace hgk {
 constexpr uint32_t kOpListMagic = 0x6f70736bu;  // "opsk"
 constexpr int kOpMaxHalf = 256;                 // rotated dims / 2
 constexpr int kOpThreads = 1024;
-constexpr int kChains = 8;                      // workgroups per token
+constexpr int kChains = 8;                      // chains per token
 
 // One op as the kernel reads it (written by the host from an hgk_op).
 struct alignas(16) DevOp {
@@ -81,13 +85,14 @@ struct alignas(16) DevOp {
   float inv_freq[kOpMaxHalf];
 };
 
-struct alignas(16) DevOpList {
+struct alignas(16) DevOpList {  // its first 16 bytes: one load
   uint32_t magic;
-  int32_t dtype;
-  int32_t count;
-  int32_t safe;         // tokens up to which the chains are independent
+  uint16_t dtype, count;  // count <= HGK_OP_LIST_MAX
+  int32_t safe;           // tokens up to which the chains are independent
+  uint16_t chains, first; // chains in use; the first op of chain 0
   DevOp ops[1];  // count entries
 };
+static_assert(HGK_OP_LIST_MAX < 65536, "count and first");
 
 constexpr int64_t op_list_bytes(int n) {
   return (int64_t)sizeof(DevOpList) + (int64_t)(n - 1) * (int64_t)sizeof(DevOp);
@@ -138,7 +143,7 @@ __device__ inline double row_sum(double v, double* part) {
 // per pass (a token's 32 head rows of 128 in one pass). rms_norm_kernel's
 // arithmetic, 16-bit X, weights in X.
 template <class X, int MODE, int G>
-__device__ void op_norm(const DevOp& op, int64_t t, double* part) {
+__device__ __forceinline__ void op_norm(const DevOp& op, int64_t t, double* part) {
   constexpr int V = Vec<X>::N;
   constexpr int P = kOpThreads / G;  // rows per pass
   const int slot = threadIdx.x / G, j = threadIdx.x % G;
@@ -212,7 +217,7 @@ __device__ void op_norm(const DevOp& op, int64_t t, double* part) {
 // 48-layer step; finding the op after next stalls on its cold descriptor.)
 // Returns the last op's index.
 template <class X, int G>
-__device__ int op_add_run(const DevOpList* list, int i, int n_ops, int64_t t, double (*part)[kOpThreads / 64]) {
+__device__ __forceinline__ int op_add_run(const DevOpList* list, int i, int n_ops, int64_t t, double (*part)[kOpThreads / 64]) {
   constexpr int V = Vec<X>::N;
   const int row = threadIdx.x / G, j = threadIdx.x % G;
   const DevOp* op = &list->ops[i];
@@ -282,7 +287,7 @@ __device__ int op_add_run(const DevOpList* list, int i, int n_ops, int64_t t, do
 }
 
 template <class X>
-__device__ int add_run_dispatch(const DevOpList* list, int i, int n_ops, int64_t t,
+__device__ __forceinline__ int add_run_dispatch(const DevOpList* list, int i, int n_ops, int64_t t,
                                 double (*part)[kOpThreads / 64]) {
   switch (list->ops[i].g) {
     case 4: return op_add_run<X, 4>(list, i, n_ops, t, part);
@@ -304,7 +309,7 @@ __device__ int add_run_dispatch(const DevOpList* list, int i, int n_ops, int64_t
 // token's position from f64 sincos, rounded to X) lives in LDS; an op whose
 // positions and frequencies are those of the previous rope op reuses it.
 template <class X, int LPR>
-__device__ void op_rope(const DevOp& op, int64_t t, bool same_table, float* cs, float* sn) {
+__device__ __forceinline__ void op_rope(const DevOp& op, int64_t t, bool same_table, float* cs, float* sn) {
   constexpr int V = Vec<X>::N;
   constexpr int P = kOpThreads / LPR;
   const int R = op.dims / (2 * V);
@@ -395,7 +400,7 @@ __device__ void op_rope(const DevOp& op, int64_t t, bool same_table, float* cs, 
 // act(gate) * up over the token's rows: one 16-byte unit per thread per pass
 // (glu_kernel's arithmetic).
 template <class X, int ACT>
-__device__ void op_glu(const DevOp& op, int64_t t) {
+__device__ __forceinline__ void op_glu(const DevOp& op, int64_t t) {
   constexpr int V = Vec<X>::N;
   const int cpr = op.n / V;
   const int total = op.rows * cpr;
@@ -424,7 +429,7 @@ __device__ void op_glu(const DevOp& op, int64_t t) {
 }
 
 template <class X, int MODE>
-__device__ void norm_dispatch(const DevOp& op, int64_t t, double* part) {
+__device__ __forceinline__ void norm_dispatch(const DevOp& op, int64_t t, double* part) {
   switch (op.g) {
     case 4: op_norm<X, MODE, 4>(op, t, part); break;
     case 8: op_norm<X, MODE, 8>(op, t, part); break;
@@ -438,62 +443,75 @@ __device__ void norm_dispatch(const DevOp& op, int64_t t, double* part) {
   }
 }
 
-template <class X>
+// ONE: a workgroup per token, which walks the chains one after another (its own
+// form: the division by `tokens` alone is 5 % of a one-op list). Else `wgs` per
+// token, workgroup wg walking chains wg, wg + wgs, ..
+template <class X, bool ONE>
 __global__ __launch_bounds__(kOpThreads) void opseq_kernel(const DevOpList* __restrict__ list,
-                                                           int n_ops, int tokens, int chained) {
+                                                           int n_ops, int tokens, int wgs) {
   __shared__ float cs[kOpMaxHalf], sn[kOpMaxHalf];
   __shared__ double part[2][kOpThreads / 64];
-  // block = (chain, token), all tokens of chain 0 (the longest) first
-  const int chain = blockIdx.x / (unsigned)tokens;
-  const int64_t t = blockIdx.x - (unsigned)chain * (unsigned)tokens;
+  // all tokens of chain 0 (the longest) first
+  if constexpr (ONE) wgs = 1;
+  const int wg = ONE ? 0 : blockIdx.x / (unsigned)tokens;
+  const int64_t t = blockIdx.x - (unsigned)wg * (unsigned)tokens;
   // a list that hgk_op_list_upload did not write for this dtype and length
   // is not walked (no pointer in it is trusted)
   if (list->magic != kOpListMagic || list->dtype != X::kCode || list->count < n_ops) return;
-  const bool serial = !chained || tokens > list->safe;  // uniform over the grid
-  if (serial && chain > 0) return;
-  // the chain's first op (the header of op c holds chain c's)
-  int i = serial ? 0 : list->ops[chain < list->count ? chain : 0].first;
-  if (chain >= list->count) i = INT32_MAX;
-  while (i < n_ops) {
-    const DevOp& op = list->ops[i];
-    if (!serial && (op.flags & kOpWait)) op_boundary();
-    int nx = serial ? i + 1 : op.next;
-    uint32_t pf[4] = {0u, 0u, 0u, 0u};
-    if (HGK_OPSEQ_PREFETCH && nx < n_ops) {
-      // one dword of each 64-byte line of the next descriptor's fields
-      const uint32_t* nd = reinterpret_cast<const uint32_t*>(&list->ops[nx]);
-      pf[0] = nd[0]; pf[1] = nd[16]; pf[2] = nd[32]; pf[3] = nd[48];
-    }
-    switch (op.kind) {
-      case kOpRms: norm_dispatch<X, kOpRms>(op, t, part[0]); break;
-      case kOpAddRms:
-        if (!serial && op.rows * op.g <= kOpThreads) {
-          nx = list->ops[add_run_dispatch<X>(list, i, n_ops, t, part)].next;
-        } else {
-          norm_dispatch<X, kOpAddRms>(op, t, part[0]);
-        }
-        break;
-      case kOpGated: norm_dispatch<X, kOpGated>(op, t, part[0]); break;
-      case kOpRope: {
-        const bool same = op.same_table & (serial ? 1 : 2);
-        switch (op.lpr) {
-          case 2: op_rope<X, 2>(op, t, same, cs, sn); break;
-          case 4: op_rope<X, 4>(op, t, same, cs, sn); break;
-          case 8: op_rope<X, 8>(op, t, same, cs, sn); break;
-          case 16: op_rope<X, 16>(op, t, same, cs, sn); break;
-          default: op_rope<X, 32>(op, t, same, cs, sn); break;
-        }
-        break;
+  const bool serial = tokens > list->safe;  // uniform over the grid
+  const int chains = serial ? 1 : list->chains;
+  // the first op of chain c is in the descriptor of op c, chain 0's in the list's header too
+  auto first = [&](int c) { return c < chains ? list->ops[c].first : INT32_MAX; };
+  int chain = wg, i = wg > 0 ? first(wg) : serial ? 0 : list->first;
+  int after = first(wg + wgs);  // where this workgroup's next chain begins
+  while (chain < chains) {
+    if (i < n_ops) {
+      const DevOp& op = list->ops[i];
+      if (!serial && (op.flags & kOpWait)) op_boundary();
+      int nx = serial ? i + 1 : op.next;
+      const int ahead = nx < n_ops ? nx : after;
+      uint32_t pf[4] = {0u, 0u, 0u, 0u};
+      if (HGK_OPSEQ_PREFETCH && ahead < n_ops) {
+        // one dword of each 64-byte line of the next descriptor's fields
+        const uint32_t* nd = reinterpret_cast<const uint32_t*>(&list->ops[ahead]);
+        pf[0] = nd[0]; pf[1] = nd[16]; pf[2] = nd[32]; pf[3] = nd[48];
       }
-      default:
-        if (op.act == HGK_ACT_SILU) op_glu<X, HGK_ACT_SILU>(op, t);
-        else op_glu<X, HGK_ACT_GELU_TANH>(op, t);
-        break;
+      switch (op.kind) {
+        case kOpRms: norm_dispatch<X, kOpRms>(op, t, part[0]); break;
+        case kOpAddRms:
+          if (!serial && op.rows * op.g <= kOpThreads) {
+            nx = list->ops[add_run_dispatch<X>(list, i, n_ops, t, part)].next;
+          } else {
+            norm_dispatch<X, kOpAddRms>(op, t, part[0]);
+          }
+          break;
+        case kOpGated: norm_dispatch<X, kOpGated>(op, t, part[0]); break;
+        case kOpRope: {
+          const bool same = op.same_table & (serial ? 1 : 2);
+          switch (op.lpr) {
+            case 2: op_rope<X, 2>(op, t, same, cs, sn); break;
+            case 4: op_rope<X, 4>(op, t, same, cs, sn); break;
+            case 8: op_rope<X, 8>(op, t, same, cs, sn); break;
+            case 16: op_rope<X, 16>(op, t, same, cs, sn); break;
+            default: op_rope<X, 32>(op, t, same, cs, sn); break;
+          }
+          break;
+        }
+        default:
+          if (op.act == HGK_ACT_SILU) op_glu<X, HGK_ACT_SILU>(op, t);
+          else op_glu<X, HGK_ACT_GELU_TANH>(op, t);
+          break;
+      }
+      if (HGK_OPSEQ_PREFETCH) asm volatile("" ::"s"(pf[0]), "s"(pf[1]), "s"(pf[2]), "s"(pf[3]));
+      if (serial) op_boundary();
+      else __syncthreads();  // the op's LDS is free
+      i = nx;
     }
-    if (HGK_OPSEQ_PREFETCH) asm volatile("" ::"s"(pf[0]), "s"(pf[1]), "s"(pf[2]), "s"(pf[3]));
-    if (serial) op_boundary();
-    else __syncthreads();  // the op's LDS is free
-    i = nx;
+    if (i >= n_ops) {
+      i = after;
+      chain += wgs;
+      after = first(chain + wgs);
+    }
   }
 }
 
@@ -843,6 +861,8 @@ void make_chains(DevOpList* L) {
       rope[c] = i;
     }
   }
+  L->chains = (uint16_t)(1 + *std::max_element(chain.begin(), chain.end()));
+  L->first = (uint16_t)L->ops[0].first;
   L->safe = (int32_t)safe;
 }
 
@@ -872,8 +892,8 @@ extern "C" int hgk_op_list_upload(int dtype, const hgk_op* ops, int n_ops, void*
   std::vector<char> host((size_t)need, 0);
   DevOpList* L = reinterpret_cast<DevOpList*>(host.data());
   L->magic = kOpListMagic;
-  L->dtype = dtype;
-  L->count = n_ops;
+  L->dtype = (uint16_t)dtype;
+  L->count = (uint16_t)n_ops;
   int last_rope = -1;
   for (int i = 0; i < n_ops; ++i) {
     const int st = translate(ops[i], i, L->ops[i]);
@@ -909,11 +929,28 @@ extern "C" int hgk_op_list_run(int dtype, const void* dev_list, int n_ops, int64
   if (tokens == 0) return HGK_OK;
   const DevOpList* L = static_cast<const DevOpList*>(dev_list);
   const dim3 b(kOpThreads);
-  // a workgroup per token and chain; where that grid would not fit, one per token
-  const int chained = tokens < ((int64_t)1 << 18);
-  const dim3 g((unsigned)(tokens * (chained ? kChains : 1)));
+  // Workgroups per token: one per chain while the tokens alone leave CUs idle. A
+  // workgroup fills a CU, so with more of them than CUs each costs a start (some
+  // 0.5 us), also where its chains are empty. us for the 192 ops of a 48-layer
+  // step / 8 independent GLUs / one add + norm, by workgroups per token:
+  //   tokens   1                 3                 4                 8
+  //   64       348 / 13.8 / 4.8  190 / 7.8 / 4.8   159 / 6.7 / 4.8   125 / 7.8 / 4.8
+  //   128      409 / 14.1 / 5.5  238 / 11.2 / 5.5  239 / 10.3 / 5.5  243 / 12.3 / 6.3
+  //   192      420 / 14.2 / 5.8  353 / 14.8 / 6.2  355 / 14.1 / 6.7  358 / 16.9 / 8.2
+  //   256      435 / 14.7 / 6.0  443 / 17.0 / 7.5  444 / 17.7 / 8.0  455 / 21.8 / 9.9
+  // and at 4096 tokens 222 / 52 us for the GLUs / the one norm against 340 / 116
+  // (one workgroup that waits after every op: 208 / 47.5; 8 adds + norms in a
+  // chain 219, 284 and 316).
+  const int wgs = tokens <= 96 ? kChains : tokens <= 128 ? 4 : tokens < 224 ? 3 : 1;
+  const dim3 g((unsigned)(tokens * wgs));
   const int nt = (int)tokens;
-  if (dtype == DT_BF16) HGK_LAUNCH((opseq_kernel<BF16>), g, b, 0, as_stream(stream), L, n_ops, nt, chained);
-  else HGK_LAUNCH((opseq_kernel<F16>), g, b, 0, as_stream(stream), L, n_ops, nt, chained);
+  const hipStream_t st = as_stream(stream);
+  if (dtype == DT_BF16) {
+    if (wgs == 1) HGK_LAUNCH((opseq_kernel<BF16, true>), g, b, 0, st, L, n_ops, nt, wgs);
+    else HGK_LAUNCH((opseq_kernel<BF16, false>), g, b, 0, st, L, n_ops, nt, wgs);
+  } else {
+    if (wgs == 1) HGK_LAUNCH((opseq_kernel<F16, true>), g, b, 0, st, L, n_ops, nt, wgs);
+    else HGK_LAUNCH((opseq_kernel<F16, false>), g, b, 0, st, L, n_ops, nt, wgs);
+  }
   return launch_status(fn);
 }

@@ -370,8 +370,15 @@ int hgk_gated_delta_gated_norm(int dtype, const void* q, const void* k, const vo
  * attention, the recurrence) are not in the list; their outputs are the ops'
  * inputs.
  *
- * One workgroup per token walks the ops in order; each op waits for the
- * previous op's stores to reach L2 before it loads. Every op is row-wise, so
+ * Ops that share bytes, one of them writing, run in list order, each after the
+ * stores of those before it; ops that share none may run in any order and side
+ * by side. hgk_op_list_upload finds out which (its host time grows in
+ * proportion to the list: 5 ms for HGK_OP_LIST_MAX ops, so upload once per set
+ * of addresses). Where ops share bytes only from some token on (views of
+ * different token strides), a run over more tokens, or any run of a list with
+ * more than 32 different token strides, takes the ops strictly in order. Where
+ * an op writes two results to the same address, the later one in the struct's
+ * order h, y stays. Every op is row-wise, so
  * token t reads only token t's rows. Results are the same bits as the
  * separate calls (hgk_rms_norm, hgk_add_rms_norm, hgk_gated_rms_norm,
  * hgk_qk_norm_rope with one position per token, hgk_glu).

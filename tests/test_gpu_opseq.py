@@ -129,6 +129,59 @@ def test_op_sequence_matches_the_separate_calls_bitwise(dev, dt, T, n_layers):
             _same_bits(g[k], r[k], f"layer {layer} {k}")
 
 
+@pytest.mark.parametrize("T,n_layers", [(96, 4), (97, 4), (129, 1), (223, 4), (224, 4), (600, 2)])
+def test_op_sequence_of_more_tokens(dev, T, n_layers):
+    """Every number of workgroups per token (8, 4, 3 and 1) gives the separate
+    calls' bits, also for the first ops of a list alone."""
+    dt = torch.bfloat16
+    L = _layers(dev, dt, T, n_layers, 74)
+    got, ref = _outputs(L, dev, dt, T), _outputs(L, dev, dt, T)
+    seq = _record(L, got, dt)
+    seq.run(T)
+    _separate(L, ref, T)
+    for layer, (g, r) in enumerate(zip(got, ref)):
+        for k in g:
+            _same_bits(g[k], r[k], f"layer {layer} {k}")
+    from higgs_amd import _lib
+    again = _outputs(L, dev, dt, T)
+    seq = _record(L, again, dt).upload()
+    _lib.check(_lib.lib().hgk_op_list_run(_lib.BF16, H.ops._ptr(seq._list), 3, T,
+                                          H.ops._stream(torch.device(dev))))
+    written = ("h_a", "y_a", "h_b", "y_b", "go")
+    for k, v in again[0].items():
+        if k in written:
+            _same_bits(v, ref[0][k], f"first ops {k}")
+        else:
+            assert bool(torch.isnan(v.float()).all()), f"{k}: written by an op past the first 3"
+
+
+def test_many_tokens_cost_one_workgroup_each(dev):
+    """A one-op list over more tokens than the chip holds workgroups: the least
+    of ten runs takes at most 7 times the separate call's (measured: 4.4 with a
+    workgroup per token, 11 with one per token and chain)."""
+    T, n, dt = 8192, 2048, torch.bfloat16
+    x, r, y = (torch.zeros(T, n, dtype=dt, device=dev) for _ in range(3))
+    seq = H.OpSequence(dt, torch.device(dev))
+    seq.glu(ACT_SILU, x, r, y)
+    seq.upload()
+
+    def least(f):
+        times = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                f()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 100)
+        return min(times[2:])
+
+    one, call = least(lambda: seq.run(T)), least(lambda: H.swiglu(x, r, out=y))
+    print(f"[opseq] {T} tokens: list {one:.1f} us, call {call:.1f} us", flush=True)
+    assert one <= 7 * call
+
+
 def test_op_sequence_residual_chain_against_the_oracle(dev):
     """Two layers' residual chain (h = x + r, y = rms_norm(h)) of the op
     sequence against the oracle's add and RMSNorm, composed on the CPU."""
