@@ -88,6 +88,36 @@ def test_tile_sizes(dev, M, N, K, ys):
     _check(got[:, :N][np.ix_(rows, cols)], ref, O.BF16, f"M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 130, 576), (500, 300, 1088), (513, 257, 192), (777, 1000, 576)],
+                         ids=["two-row-blocks", "eight", "hi-lo", "hi-lo-ragged"])
+def test_other_k_over_many_rows(dev, M, N, K):
+    """K that is no multiple of 512: the exact-product kernel up to 512 rows, the
+    hi/lo-plane kernel above (weights to 2^-17, well inside the bar)."""
+    x, w, s, b = _case(4201 + M + N, M, N, K)
+    got = _run(dev, x, w, s, b, O.BF16)
+    ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
+    _check(got, ref, O.BF16, f"M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 70, 3584), (9, 200, 2048), (64, 300, 2048), (100, 384, 512),
+                                   (600, 200, 1024)],
+                         ids=["one-row", "few-rows", "decode", "exact", "hi-lo"])
+def test_scales_off_a_word_boundary(dev, M, N, K):
+    """Scales and biases that start at an odd element: the kernels that load them
+    4 or 16 bytes at a time leave the call to the others."""
+    x, w, s, b = _case(4301 + M + N, M, N, K)
+
+    def odd(a):
+        t = torch.empty(a.size + 1, dtype=torch.bfloat16, device=dev)
+        t[1:] = to_dev(a, O.BF16, dev).flatten()
+        assert t[1:].data_ptr() % 4 == 2
+        return t[1:].view(a.shape)
+
+    got = to_host(H.quantized_matmul(to_dev(x, O.BF16, dev), words_dev(w, dev), odd(s), odd(b)))
+    ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
+    _check(got, ref, O.BF16, f"odd scales M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("M,N,K", [(33, 512, 2048), (64, 4096, 2048), (40, 8200, 2048),
                                    (129, 200, 1024), (301, 1001, 512), (1024, 2048, 512),
                                    (700, 12288, 512), (4100, 12288, 512)],
