@@ -664,8 +664,8 @@ def wl_qwen3_next_decode(cx):
 
 def wl_qwen3_next_decode_opseq(cx):
     """The same 48-layer op sequence (same ops, same buffers) in one launch:
-    one workgroup per sequence walks the 192 ops in the layer loop's order,
-    each op waiting for the previous op's stores (hgk_op_list_run)."""
+    a workgroup per sequence and chain of dependent ops walks the chain in the
+    layer loop's order (hgk_op_list_run)."""
     from higgs_amd.ops import OpSequence
     torch = cx.torch
     S = 64

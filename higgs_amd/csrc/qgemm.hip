@@ -4,10 +4,11 @@
 // with w [N, K/8] u32 (8 codes per word, low nibble first) and scales/biases
 // [N, K/64] in the activation dtype (bf16).
 //
-// Four kernels: the decode kernel for M <= 64 with K a multiple of 512
-// (further down), the tiles of qgemm_tile.hip for more rows of such K, and
-// for other K (or operands those do not take) the exact-product kernel below
-// (M <= 512) and the hi/lo-plane kernel (M > 512).
+// Four kernels: with K a multiple of 512 the decode kernel (further down) for
+// 16 to 64 rows, and for 2 to 15 where qgemm_few_rows_fits; the tiles of
+// qgemm_tile.hip for more rows, and for 33 to 64 over few columns; for other K
+// (or operands those do not take) the exact-product kernel below (M <= 512) and
+// the hi/lo-plane kernel (M > 512). qgemm.h says what fewer rows run on.
 //
 // Exact products, one group at a time. A code q enters the matrix core as
 // the bf16 number 128 + q (two bit operations per pair of codes), x as

@@ -4,7 +4,8 @@
 // Exact products: a code q enters the matrix core as the bf16 number q, so
 // every product x q is exact, and per 64-code group acc += s * C with
 // C = sum x q in f32. The bias term sum_g b Sx_g, with the row sums Sx_g of
-// x, is one more bf16 MFMA per tile and 4 groups: Sx_g is split into three
+// x (ones against x: every column of that product is one row's own), is one
+// more bf16 MFMA per tile and 4 groups: Sx_g is split into three
 // bf16 parts (24 bits: nothing is rounded), b is a bf16 number already, and
 // the 16 k-slots of the MFMA take 4 groups x 3 such products.
 //
@@ -502,7 +503,9 @@ bool qgemm_tile_fits(const QgemmArgs& a) {
 // 36.5 / 17.3, 4096 x 4096 20.2 / 11.4, 2048 x 2048 10.8 / 7.2; 33 rows 37.9 /
 // 26.3, 24.6 / 16.4, 14.3 / 11.0, 7.7 / 7.1. Up to 32 rows the decode kernel is
 // as fast or faster (17 rows, 2048 x 2048: 6.0 / 7.0), and so it is with more
-// columns (64 rows, 12288 x 4096: 22.6 / 31.8).
+// columns where 96-column tiles fill one round of CUs (64 rows, 12288 x 4096:
+// 22.6 / 31.8). Past that it is not (64 rows, 14336 x 3584: 39.3, 23.7 in this
+// arithmetic): those calls stay on the decode kernel for want of a rule.
 bool qgemm_tile_split_fits(const QgemmArgs& a) {
   return a.M > 32 && a.M <= 64 && a.K % 2048 == 0 && 2 * ((a.N + 31) / 32) <= 256 && qgemm_tile_fits(a);
 }

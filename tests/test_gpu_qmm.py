@@ -269,8 +269,8 @@ def test_grouped_partial_column_tiles(dev, N):
 
 def test_grouped_size_with_unaligned_pair_count(dev):
     """A pair count that is not a multiple of 4 (the grouped kernel reads the
-    expert ids 16 bytes at a time, so it leaves such a call to the per-pair
-    kernel) gives the oracle's result, including the last pairs."""
+    expert ids 16 bytes at a time and the last ones one by one) gives the
+    oracle's result, including the last pairs."""
     P, R, E, N, K = 4098, 600, 8, 128, 512
     x, w, s, b, ex = _case(2421, P, R, E, N, K)
     got = _run(dev, x, w, s, b, ex, O.BF16, x_div=7)
