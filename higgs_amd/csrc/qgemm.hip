@@ -1494,20 +1494,28 @@ bool gather_xp_fits(const GatherArgs& a) {
 // 264 us, gate 355 -> 126 (128 and 64 blocks before, 512 and 320 now). With a
 // block per CU already, parts gained nothing (8 of 128 experts, 2048 -> 1024:
 // gate 224 us, 259 in two parts): each part reads the weights again.
+struct XpGrid {
+  int64_t gx, tpg, gz;  // blocks and column tiles of a block, parts
+};
+XpGrid xp_grid(const GatherArgs& a, int bno) {
+  const int64_t ntiles = (a.N + bno - 1) / bno;
+  XpGrid g;
+  g.gx = 1024 / (a.E + 1);
+  g.gx = g.gx < 1 ? 1 : (g.gx > ntiles ? ntiles : g.gx);
+  g.tpg = (ntiles + g.gx - 1) / g.gx;
+  g.gx = (ntiles + g.tpg - 1) / g.tpg;
+  g.gz = 1;
+  if (a.E * g.gx < kCUs) {
+    const int64_t fill = 2 * kCUs / (a.E * g.gx), full = a.pairs / (a.E * 16 * HGK_XP_RT);
+    g.gz = fill < full ? fill : full;
+    g.gz = g.gz < 1 ? 1 : g.gz;
+  }
+  return g;
+}
+
 template <bool SW>
 void gather_xp_launch(const GatherArgs& a, hipStream_t s) {
-  constexpr int BNO = SW ? kXpBN / 2 : kXpBN;
-  const int64_t ntiles = (a.N + BNO - 1) / BNO;
-  int64_t gx = 1024 / (a.E + 1);
-  gx = gx < 1 ? 1 : (gx > ntiles ? ntiles : gx);
-  const int64_t tpg = (ntiles + gx - 1) / gx;
-  gx = (ntiles + tpg - 1) / tpg;
-  int64_t gz = 1;
-  if (a.E * gx < kCUs) {
-    const int64_t fill = 2 * kCUs / (a.E * gx), full = a.pairs / (a.E * 16 * HGK_XP_RT);
-    gz = fill < full ? fill : full;
-    gz = gz < 1 ? 1 : gz;
-  }
+  const auto [gx, tpg, gz] = xp_grid(a, SW ? kXpBN / 2 : kXpBN);
   const int64_t part = ((a.pairs + gz - 1) / gz + 3) / 4 * 4;
   const dim3 grid((unsigned)gx, (unsigned)(a.E + 1), (unsigned)((a.pairs + part - 1) / part));
   if constexpr (!SW) {
@@ -1524,8 +1532,23 @@ void gather_xp_launch(const GatherArgs& a, hipStream_t s) {
 
 // A pair count that is no multiple of 4: where the per-pair GEMV has K, which
 // this form's sums are no less exact than (other K sum x (s q + b) per pair).
+// And where it is faster: a pass of a block takes about 5 us and, per 64 codes
+// of K, 1.2 us and 0.17 per row tile; the per-pair kernel reads some 17e12
+// codes per second. us, per pair / grouped (experts, K -> N, pairs):
+//   8, 2048 -> 512    130 13.7 / 42.8   514 36.8 / 62.4   1602 105 / 179
+//   8, 512 -> 2048    162 14.3 / 16.9   258 20.7 / 18.4   1602 108 / 48
+//   64, 2048 -> 512   1026 66.9 / 46.4  4098 242 / 70     12802 680 / 185
+//   4, 1024 -> 300    66 5.3 / 24.3     802 19.4 / 81
+//   2, 4096 -> 1024   34 20.4 / 78.3    402 122 / 273
 bool gather_ragged_fits(const GatherArgs& a) {
-  return HGK_GATHER_XP && (a.K == 512 || a.K == 1024 || a.K == 2048 || a.K == 4096) && gather_xp_fits(a);
+  if (!HGK_GATHER_XP || (a.K != 512 && a.K != 1024 && a.K != 2048 && a.K != 4096) || !gather_xp_fits(a)) return false;
+  const XpGrid g = xp_grid(a, kXpBN);
+  const int64_t rows = (a.pairs + a.E * g.gz - 1) / (a.E * g.gz);  // of a block, on average
+  const int64_t passes = g.tpg * ((rows + 16 * HGK_XP_RT - 1) / (16 * HGK_XP_RT));
+  const int64_t rounds = (a.E * g.gx * g.gz + kCUs - 1) / kCUs;
+  const int64_t rt = rows < 16 * HGK_XP_RT ? (rows + 15) / 16 : HGK_XP_RT;
+  const double grouped = rounds * passes * (5.0 + a.K / 64 * (1.2 + 0.17 * rt));
+  return grouped < 3.0 + (double)a.pairs * a.N * a.K * 5.9e-8;
 }
 
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s) {

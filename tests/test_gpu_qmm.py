@@ -239,12 +239,12 @@ def test_grouped_hilo_path_for_other_k(dev):
 def test_grouped_path_routing_and_out_of_range(dev):
     """The grouped kernel keeps gather_qmm's routing rules: lhs rows, -1
     wrapping to the last expert, out-of-range experts and rows giving zero
-    rows; one expert with more pairs than one scan pass lists (the list is
-    drained and the scan resumes)."""
+    rows; few experts, one of them with 9000 pairs, so that the pairs are split
+    over several blocks."""
     P, R, E, N, K = 10000, 40, 4, 128, 512
     x, w, s, b, ex = _case(2411, P, R, E, N, K)
     ex = ex.copy()
-    ex[:9000] = 1                  # 9000 pairs on one expert: the list fills and drains
+    ex[:9000] = 1
     ex[[5, 2300]] = [E + 2, -1]    # out of range -> zero row; -1 wraps to E - 1
     lhs = (np.arange(P) * 13) % R
     lhs[7] = R                     # row out of range -> zero row
@@ -268,9 +268,9 @@ def test_grouped_partial_column_tiles(dev, N):
 
 
 def test_grouped_size_with_unaligned_pair_count(dev):
-    """A pair count that is not a multiple of 4 (the grouped kernel reads the
-    expert ids 16 bytes at a time and the last ones one by one) gives the
-    oracle's result, including the last pairs."""
+    """A pair count that is not a multiple of 4, few experts and few columns (the
+    per-pair kernel is the faster one) gives the oracle's result, including the
+    last pairs."""
     P, R, E, N, K = 4098, 600, 8, 128, 512
     x, w, s, b, ex = _case(2421, P, R, E, N, K)
     got = _run(dev, x, w, s, b, ex, O.BF16, x_div=7)
@@ -283,9 +283,10 @@ def test_grouped_size_with_unaligned_pair_count(dev):
                          ids=["one-past-a-round", "three", "two-long-lists", "other-K"])
 def test_grouped_last_pairs_and_parts(dev, P, K):
     """Pair counts that end 1, 2 or 3 past a 16-byte read of the ids, with few
-    experts (their pairs are split over several blocks where K is a multiple
-    of 512), one of them taking half of all pairs, and ids out of range."""
-    R, E, N = 400, 4, 200
+    experts (K 512: the grouped kernel, their pairs split over several blocks;
+    K 576: per pair), one of them taking half of all pairs, and ids out of
+    range."""
+    R, E, N = 400, 4, 520
     x, w, s, b, ex = _case(2481 + P, P, R, E, N, K)
     ex[::2] = 1
     ex[[5, P - 1]] = [E, -E - 1]
@@ -299,23 +300,24 @@ def test_grouped_last_pairs_and_parts(dev, P, K):
 
 
 @pytest.mark.parametrize("P,K", [(20000, 512), (20002, 512), (16384, 576)],
-                         ids=["parts", "ragged", "other-K"])
+                         ids=["usual", "ragged", "other-K"])
 def test_grouped_list_that_fills_again_and_again(dev, P, K):
-    """Nearly all pairs on one expert of two, so that a block's list of pairs
+    """Nearly all pairs on one expert of 300, so that its block's list of pairs
     fills, is drained and fills again: every pair is computed once, to the bits
     of the other pairs with the same row and expert."""
-    R, E, N = 37, 2, 72
+    R, E, N = 37, 300, 136  # enough experts that the pairs are not split in parts
     x, w, s, b, ex = _case(2541 + P, P, R, E, N, K)
-    ex = np.ones_like(ex)
-    ex[::997] = 0
+    ex = np.full_like(ex, 7)
+    ex[::997] = 299
     lhs = (np.arange(P) % R).astype(np.int32)
     got = _run(dev, x, w, s, b, ex, O.BF16, lhs=lhs)
-    want = O.gather_qmm(x, O.BF16, w, s, b, O.BF16, np.repeat([0, 1], R).astype(np.int32),
+    which = (ex == 299).astype(np.int64)
+    want = O.gather_qmm(x, O.BF16, w, s, b, O.BF16, np.repeat([7, 299], R).astype(np.int32),
                         lhs=np.tile(np.arange(R), 2).astype(np.int32)).reshape(2, R, N)
-    one = np.stack([[got[np.flatnonzero((ex == e) & (lhs == r))[0]] if ((ex == e) & (lhs == r)).any()
+    one = np.stack([[got[np.flatnonzero((which == e) & (lhs == r))[0]] if ((which == e) & (lhs == r)).any()
                      else want[e, r] for r in range(R)] for e in (0, 1)])
     _check(one, want, O.BF16, f"long list P={P} K={K}")
-    assert np.array_equal(got, one[ex, lhs])
+    assert np.array_equal(got, one[which, lhs])
 
 
 @pytest.mark.parametrize("mean", [0.0, 1.0])
