@@ -55,20 +55,14 @@ void gather_grouped_launch(const GatherArgs& a, hipStream_t s);
 bool gather_swiglu_grouped_launch(const GatherArgs& a, hipStream_t s);
 
 // Rows of x at or above which the MFMA kernels run for every K. Below:
-// - 2 to 15 rows where the one-row GEMV has K (512, 1024, 2048 or 4096): the
-//   decode kernel's form for few rows, which reads each weight once for all of
-//   them; its f32 sums are no less exact than the GEMV's (see there);
-// - one row: the GEMV;
+// - one row: the one-row GEMV (K 512, 1024, 2048 and 4096);
+// - 2 to 15 rows of these K: the decode kernel's form for few rows where it is
+//   faster (qgemm_few_rows_fits), which reads each weight once for all rows and
+//   whose f32 sums are no less exact than the GEMV's; else the GEMV, row by row;
 // - other K: qmv_chain_kernel or the generic kernel (qmm.hip), whose sums of
 //   x (s q + b) no group form reaches where x has a mean.
-// us per call, GEMV / decode kernel:
-//   N x K           1 row         4 rows        15 rows
-//   12288 x 4096    12.6 / 11.6   23.5 / 12.2   60.5 / 13.5
-//   12288 x 2048    6.3 / 6.5     10.1 / 6.7    25.4 / 7.2
-//   4096 x 4096     9.7 / 7.9     10.1 / 8.1    23.9 / 9.6
-//   2048 x 2048     5.4 / 5.9     5.4 / 6.0     7.4 / 5.8
-// (One row is 8 to 20 % slower with K 4096 than on the decode kernel, and
-// gives the bits that gather_qmm gives for the same row.)
+// (One row of K 4096 is 8 to 20 % slower than on the decode kernel, 12.6 / 11.6
+// us at 12288 x 4096, and gives the bits that gather_qmm gives for the row.)
 constexpr int64_t kQgemmMinRows = 16;
 
 // bf16 activations and scales, group 64, 4 bits, x 16-byte aligned with a

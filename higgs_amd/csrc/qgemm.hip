@@ -1641,8 +1641,27 @@ bool qgemm_supported(int dtype, int sdt, int group_size, int bits, const void* x
          (reinterpret_cast<uintptr_t>(w) & 7) == 0 && ((k / 8) % 2) == 0;
 }
 
+// The few-row form where it is the faster side. The GEMV runs its rows side by
+// side, so it takes one row's time until the blocks of all rows fill the chip;
+// long rows make that time. us, GEMV / few-row form (N x K):
+//   K 4096  2 rows  4096 9.8 / 7.7   9000 17.2 / 12.2  16384 18.4 / 17.2
+//   K 2048  2 rows  4096 5.4 / 4.7   9000 8.9 / 6.8    16384 8.7 / 9.2, 3 rows 10.4 / 9.1
+//   K 1024  2 rows  4096 3.5 / 3.9   9000 5.6 / 5.4    16384 5.6 / 7.0
+//           5 rows  2048 3.5 / 4.0   4096 4.4 / 4.1    16384 8.0 / 7.2
+//   K 512   5 rows  4096 3.3 / 3.8   9000 5.2 / 4.7    16384 5.4 / 6.5
+//           8 rows  4096 3.3 / 3.9   9000 6.4 / 4.8    16384 6.7 / 6.6
+bool few_rows_faster(const QgemmArgs& a) {
+  switch (a.K) {
+    case 4096: return a.M >= 2;
+    case 2048: return a.M >= 3 || (a.M == 2 && a.N <= 48 * kCUs);
+    case 1024: return a.M >= 5 && a.M * a.N >= 20000;
+    case 512: return a.M >= 8 && a.M * a.N >= 60000;
+    default: return false;
+  }
+}
+
 bool qgemm_few_rows_fits(const QgemmArgs& a) {
-  return a.M > 1 && (a.K == 512 || a.K == 1024 || a.K == 2048 || a.K == 4096) && decode_fits(a) &&
+  return few_rows_faster(a) && decode_fits(a) &&
          (reinterpret_cast<uintptr_t>(a.w) & 15) == 0 &&
          ((reinterpret_cast<uintptr_t>(a.sc) | reinterpret_cast<uintptr_t>(a.bi)) & 3) == 0;
 }

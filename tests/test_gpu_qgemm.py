@@ -200,10 +200,11 @@ def test_decode_rows_over_few_columns(dev, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 17, 512), (1, 4096, 3584), (2, 1000, 2048), (1, 512, 12288),
-                                   (15, 64, 8192), (7, 12289, 512)])
+                                   (15, 64, 8192), (7, 12289, 512), (2, 12288, 2048), (2, 12289, 2048),
+                                   (5, 4000, 1024), (4, 5100, 1024), (8, 7500, 512), (7, 8600, 512)])
 def test_few_rows_of_any_k(dev, M, N, K):
     """1 to 15 rows: column tiles that are partly filled, K beyond the GEMV's
-    list, few and many column tiles."""
+    list, few and many column tiles, both sides of the rules for few rows."""
     x, w, s, b = _case(3901 + M + N, M, N, K)
     got = _run(dev, x, w, s, b, O.BF16)
     ref = O.quantized_matmul(x, O.BF16, w, s, b, O.BF16)
