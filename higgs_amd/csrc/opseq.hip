@@ -646,9 +646,8 @@ int64_t first_overlap(Range a, Range b) {
   return d0 + t * dt < a.span ? t : INT64_MAX;
 }
 
-// An op's ranges; range 0 is x.
-std::vector<Range> op_ranges(const DevOp& d, int op, std::map<std::array<int64_t, 5>, int>& keys) {
-  std::vector<Range> v;
+// Append an op's ranges to v; x is the first.
+void op_ranges(const DevOp& d, int op, std::map<std::array<int64_t, 5>, int>& keys, std::vector<Range>& v) {
   const bool own = d.kind == kOpAddRms && d.rows * d.g <= kOpThreads;
   auto add = [&](const void* p, int64_t tok, int64_t rows, int64_t row, bool write) {
     if (!p || rows <= 0) return;
@@ -677,7 +676,6 @@ std::vector<Range> op_ranges(const DevOp& d, int op, std::map<std::array<int64_t
     if (d.w2) other(d.w2, 0, d.n * 2, 0);
     if (d.offsets) other(d.offsets, 0, 4, 4);
   }
-  return v;
 }
 
 struct Groups {
@@ -699,16 +697,15 @@ struct Groups {
 };
 
 // Join the ops that share bytes of token 0, one of them writing: a sweep over
-// the ranges by address. Of the writes that reach the current address one
+// the ranges, sorted by address. Of the writes that reach the current address one
 // stands for all (they overlap there, so their ops are joined; the one that
 // ends last is met by whatever meets any), and so does one of the reads that a
 // write has joined.
-void join_overlaps(std::vector<Range> all, Groups& g) {
-  std::sort(all.begin(), all.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
+void join_overlaps(const std::vector<Range>& sorted, Groups& g) {
   Range w{};  // the write that ends last (op -1: none)
   w.op = -1;
   std::vector<Range> reads;  // not joined with each other; some have ended
-  for (const Range& r : all) {
+  for (const Range& r : sorted) {
     if (w.op >= 0 && w.end() > r.lo) g.join(w.op, r.op);
     if (!r.write) {
       reads.push_back(r);
@@ -731,16 +728,15 @@ void join_overlaps(std::vector<Range> all, Groups& g) {
 // or `safe` where that is smaller. Per pair of strides, each range of the
 // larger one meets the ranges above it, nearest first, until a range is too far
 // to be met before `safe`.
-int64_t first_later_overlap(const std::vector<Range>& all, int64_t safe) {
+int64_t first_later_overlap(const std::vector<Range>& sorted, int64_t safe) {
   std::map<int64_t, std::array<std::vector<Range>, 2>> by;  // per stride: all ranges, the writes
-  for (const Range& r : all) {
-    by[r.tok][0].push_back(r);
-    if (r.write) by[r.tok][1].push_back(r);
+  for (const Range& r : sorted) {
+    auto& lists = by[r.tok];
+    lists[0].push_back(r);
+    if (r.write) lists[1].push_back(r);
   }
   // (many strides would make many pairs: such a list runs in order)
   if (by.size() > 32) return 0;
-  for (auto& [tok, lists] : by)
-    for (auto& l : lists) std::sort(l.begin(), l.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
   for (const auto& [small, as] : by)
     for (const auto& [large, bs] : by) {
       if (large <= small) continue;
@@ -785,15 +781,18 @@ struct Touched {
 void make_chains(DevOpList* L) {
   const int n = L->count;
   std::map<std::array<int64_t, 5>, int> keys;
-  std::vector<std::vector<Range>> rg(n);
-  std::vector<Range> all;
+  std::vector<Range> all;        // op i's ranges: at[i] .. at[i + 1] - 1
+  std::vector<size_t> at(n + 1, 0);
+  all.reserve(6 * n);
   for (int i = 0; i < n; ++i) {
-    rg[i] = op_ranges(L->ops[i], i, keys);
-    all.insert(all.end(), rg[i].begin(), rg[i].end());
+    op_ranges(L->ops[i], i, keys, all);
+    at[i + 1] = all.size();
   }
+  std::vector<Range> sorted = all;
+  std::sort(sorted.begin(), sorted.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
   Groups groups(n);
-  join_overlaps(all, groups);
-  int64_t safe = first_later_overlap(all, INT32_MAX);
+  join_overlaps(sorted, groups);
+  int64_t safe = first_later_overlap(sorted, INT32_MAX);
   // the largest group of dependent ops is chain 0; each other group goes to
   // the chain with the fewest ops so far
   int big = 0;
@@ -833,15 +832,15 @@ void make_chains(DevOpList* L) {
       // where q's y lies on its h, x is y, stored last
       int64_t over = INT64_MAX;
       if (carry)
-        for (const Range& a : rg[p])
-          for (const Range& b : rg[p])
-            if (a.write && b.write && &a < &b) over = std::min(over, first_overlap(a, b));
+        for (size_t a = at[p]; a < at[p + 1]; ++a)
+          for (size_t b = a + 1; b < at[p + 1]; ++b)
+            if (all[a].write && all[b].write) over = std::min(over, first_overlap(all[a], all[b]));
       carry = carry && over > 0;
       // a carried op reads x from registers, and where it writes what the same
       // threads read or wrote before, program order is enough
       bool wait = false;
-      for (size_t k = carry ? 1 : 0; k < rg[i].size() && !wait; ++k) {
-        const Range& r = rg[i][k];
+      for (size_t k = at[i] + carry; k < at[i + 1] && !wait; ++k) {
+        const Range& r = all[k];
         const int but = carry && r.write ? r.key : -1;
         wait = writes[c].meets(r, but) || (r.write && reads[c].meets(r, but));
       }
@@ -851,10 +850,11 @@ void make_chains(DevOpList* L) {
       }
       if (wait) {
         d.flags |= kOpWait;
-        reads[c] = writes[c] = Touched();
+        reads[c].seg.clear();
+        writes[c].seg.clear();
       }
     }
-    for (const Range& r : rg[i]) (r.write ? writes : reads)[c].add(r);
+    for (size_t k = at[i]; k < at[i + 1]; ++k) (all[k].write ? writes : reads)[c].add(all[k]);
     last[c] = i;
     if (d.kind == kOpRope) {
       if (rope[c] >= 0 && same_positions(L->ops[rope[c]], d)) d.same_table |= 2;
